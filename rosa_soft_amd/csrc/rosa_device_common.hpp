@@ -77,6 +77,24 @@ __device__ __forceinline__ float wave_max_lane63(float v) {
   return v;
 }
 
+// Minimum over the 64 lanes; the result is valid in lane 63 only.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ uint32_t dpp_min(uint32_t acc) {
+  const uint32_t moved = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+      static_cast<int>(acc), static_cast<int>(acc), CTRL, ROW_MASK, 0xf, false));
+  return min(acc, moved);
+}
+
+__device__ __forceinline__ uint32_t wave_min_lane63(uint32_t v) {
+  v = dpp_min<0x111, 0xf>(v);
+  v = dpp_min<0x112, 0xf>(v);
+  v = dpp_min<0x114, 0xf>(v);
+  v = dpp_min<0x118, 0xf>(v);
+  v = dpp_min<0x142, 0xa>(v);
+  v = dpp_min<0x143, 0xc>(v);
+  return v;
+}
+
 // A wave-uniform value as a vector register.  Simple vector instructions (add, multiply,
 // fma, logic, right shifts) issue at twice the rate of the others on gfx950 when two waves
 // share a SIMD, but not when one of their operands is a scalar register: constants of the
@@ -249,6 +267,41 @@ __host__ __device__ inline int64_t checkpoint_slots(int64_t steps, int64_t bands
   return steps / 16 + bands + 1;
 }
 
+// Rows of a piece of a band (a multiple of `align`), 0 for whole bands: `band_rows` rows of all
+// bands together over `capacity` resident waves is what every wave would walk if the work
+// could be cut anywhere, and bands longer than that are cut into equal pieces of about that
+// length.  Never below `least` rows: what a piece costs beyond its own rows (the sweep in front
+// of it, the halo below it) is of that size.
+__host__ __device__ inline int piece_rows_for(int64_t band_rows, int longest, int64_t capacity,
+                                              int least, int align) {
+  const int64_t share = (band_rows + capacity - 1) / capacity;
+  const int64_t ideal = share > least ? share : least;
+  if (longest - 1 <= ideal) return 0;
+  const int64_t pieces = (longest - 1 + ideal - 1) / ideal;
+  const int64_t rows = (longest - 1 + pieces - 1) / pieces;
+  return static_cast<int>((rows + align - 1) / align * align);
+}
+
+__host__ __device__ inline int pieces_of_band(int piece_rows, int longest) {
+  return piece_rows > 0 && longest > 1 ? (longest - 1 + piece_rows - 1) / piece_rows : 1;
+}
+
+// Bands of a sequence of `len` tokens that have a piece number `piece` (band j has
+// len - 1 - 64 j rows), and pieces of all its bands.
+__host__ __device__ inline int bands_with_piece(int len, int piece_rows, int piece) {
+  const int64_t rows_left = static_cast<int64_t>(len) - 1 - static_cast<int64_t>(piece) * piece_rows;
+  return rows_left > 0 ? static_cast<int>((rows_left + 63) / 64) : 0;
+}
+
+__host__ __device__ inline int64_t pieces_of_sequence(int len, int piece_rows) {
+  int64_t pieces = 0;
+  for (int piece = 0;; ++piece) {
+    const int bands = bands_with_piece(len, piece_rows, piece);
+    pieces += bands;
+    if (bands == 0 || piece_rows <= 0) return pieces;
+  }
+}
+
 struct Unit {
   int seq;     // batch index (dense) or packed sequence index
   int block;   // 64-row block / 64-diagonal band index inside the sequence
@@ -259,8 +312,82 @@ struct Unit {
   bool valid;
 };
 
-// slot order is block-major so that equal block indices of all sequences are adjacent
+// A value of the packed-sequence tables, the same in every lane of the wave.  The tables are
+// written by a kernel of the same stream, so the compiler reads them with vector loads and
+// keeps everything derived from them, addresses included, in vector registers.  SCALAR moves
+// the value to scalar registers, for kernels that are short of vector registers (thirty fewer
+// in the gradient kernel); its two-wave form is short of scalar ones and was 4 % slower for it.
+template <bool SCALAR>
+__device__ __forceinline__ int table_value(int value) {
+  return SCALAR ? __builtin_amdgcn_readfirstlane(value) : value;
+}
+
+template <bool SCALAR>
+__device__ __forceinline__ int64_t table_value(int64_t value) {
+  if constexpr (!SCALAR) return value;
+  const uint32_t low = __builtin_amdgcn_readfirstlane(static_cast<int>(value));
+  const uint32_t high = __builtin_amdgcn_readfirstlane(static_cast<int>(value >> 32));
+  return static_cast<int64_t>(static_cast<uint64_t>(high) << 32 | low);
+}
+
+// Work item `index` of bands cut into pieces, numbered without gaps: piece 0 of every band,
+// then piece 1 of the bands long enough to have one, and so on (in a packed batch sequence by
+// sequence, `item_prefix` items before each).  Items that turn out to be empty are not free: a
+// wave pays for each with a pull from the work counter, and pulls come one at a time (40 ns).
 template <bool VARLEN>
+__device__ __forceinline__ Unit decode_piece(const Layout& L, const int32_t* item_prefix,
+                                             int piece_rows, int index, int& piece) {
+  Unit u;
+  u.valid = true;
+  int local = index, copies = L.B * L.H;
+  if constexpr (VARLEN) {
+    int low = 0, high = L.S;  // find seq with prefix[seq] <= index < prefix[seq+1]
+    while (low < high) {
+      const int mid = (low + high) >> 1;
+      if (table_value<true>(item_prefix[mid + 1]) <= index) low = mid + 1; else high = mid;
+    }
+    if (low >= L.S) {
+      u.valid = false;
+      u.seq = 0; u.block = 0; u.start = 0; u.len = 0; u.head = 0; u.word_base = 0;
+      piece = 0;
+      return u;
+    }
+    u.seq = low;
+    local = index - table_value<true>(item_prefix[low]);
+    copies = L.H;
+    u.start = table_value<true>(L.seq_start[low]);
+    u.len = table_value<true>(L.seq_len[low]);
+  } else {
+    u.len = L.T;
+  }
+  piece = 0;
+  for (;;) {
+    const int here = bands_with_piece(u.len, piece_rows, piece) * copies;
+    if (local < here) break;
+    if (here == 0) {  // (dense: beyond the last item)
+      u.valid = false;
+      u.seq = 0; u.block = 0; u.start = 0; u.len = 0; u.head = 0; u.word_base = 0;
+      return u;
+    }
+    local -= here;
+    ++piece;
+  }
+  u.block = local / copies;
+  local -= u.block * copies;
+  if constexpr (VARLEN) {
+    u.head = local;
+    u.word_base = static_cast<int64_t>(u.head) * L.N + u.start;
+  } else {
+    u.seq = local / L.H;
+    u.head = local - u.seq * L.H;
+    u.start = u.seq * L.T;
+    u.word_base = (static_cast<int64_t>(u.seq) * L.H + u.head) * L.T;
+  }
+  return u;
+}
+
+// slot order is block-major so that equal block indices of all sequences are adjacent
+template <bool VARLEN, bool SCALAR = false>
 __device__ __forceinline__ Unit decode_unit(const Layout& L, int unit_index) {
   Unit u;
   u.head = unit_index % L.H;
@@ -270,7 +397,7 @@ __device__ __forceinline__ Unit decode_unit(const Layout& L, int unit_index) {
     int low = 0, high = L.S;  // find seq with prefix[seq] <= slot < prefix[seq+1]
     while (low < high) {
       const int mid = (low + high) >> 1;
-      if (L.block_prefix[mid + 1] <= slot) low = mid + 1; else high = mid;
+      if (table_value<SCALAR>(L.block_prefix[mid + 1]) <= slot) low = mid + 1; else high = mid;
     }
     if (low >= L.S) {
       u.valid = false;
@@ -278,9 +405,9 @@ __device__ __forceinline__ Unit decode_unit(const Layout& L, int unit_index) {
       return u;
     }
     u.seq = low;
-    u.block = slot - L.block_prefix[low];
-    u.start = L.seq_start[low];
-    u.len = L.seq_len[low];
+    u.block = slot - table_value<SCALAR>(L.block_prefix[low]);
+    u.start = table_value<SCALAR>(L.seq_start[low]);
+    u.len = table_value<SCALAR>(L.seq_len[low]);
     u.word_base = static_cast<int64_t>(u.head) * L.N + u.start;
   } else {
     u.seq = slot % L.B;

@@ -79,13 +79,24 @@ void stage_end(Stage stage, hipStream_t stream) {
 // packed-sequence table: sanitised offsets and block prefix sums
 // ---------------------------------------------------------------------------
 
+// How the bands of a packed batch may be cut (the host knows neither their lengths nor,
+// therefore, their number): waves of the two passes that run at a time, and the rows of a piece
+// the caller insists on (0: by shape, negative: whole bands).
+struct PieceLimits {
+  int64_t gradient_waves, stats_waves;
+  int forced_gradient_rows;
+  int64_t stats_items_most;     // work items the grid of the row-statistics kernel has room for
+  int32_t* gradient_prefix;     // [S + 1] pieces before each sequence, of either pass
+  int32_t* stats_prefix;
+};
+
 __global__ void prepare_sequences_kernel(const int32_t* __restrict__ cu_seqlens, int S, int N,
                                          int32_t* __restrict__ seq_start,
                                          int32_t* __restrict__ seq_len,
                                          int32_t* __restrict__ block_prefix,
                                          int64_t* __restrict__ step_prefix, int H,
                                          int64_t checkpoint_capacity,
-                                         int32_t* __restrict__ header) {
+                                         int32_t* __restrict__ header, PieceLimits pieces) {
   // Single block.  Offsets are valid iff they start at 0, end at N and never decrease.
   // When they are not, every sequence is made empty, so that no later kernel touches a
   // token, and header[0] is set: the kernels that write results then fill them with NaN.
@@ -124,16 +135,75 @@ __global__ void prepare_sequences_kernel(const int32_t* __restrict__ cu_seqlens,
     header[0] = bad;
   }
   __syncthreads();
-  if (threadIdx.x == 0 && step_prefix != nullptr) {
-    // index space of the chunk records; they are used only if they fit
+  if (step_prefix != nullptr) {
+    // Index space of the chunk records, and the pieces of the bands: every thread takes its own
+    // run of sequences, and the first one adds up what the threads have found.
+    __shared__ int64_t sums[3][256];
+    __shared__ int longest_of[256];
+    __shared__ int plan[2];
     int64_t steps = 0;
-    for (int s = 0; s < S; ++s) {
-      step_prefix[s] = steps;
+    int longest = 0;
+    for (int s = first; s < last; ++s) {
       steps += band_steps_total(seq_len[s]);
+      longest = max(longest, seq_len[s]);
     }
-    step_prefix[S] = steps;
-    header[3] = checkpoint_slots(steps * H, static_cast<int64_t>(block_prefix[S]) * H) <=
-                        checkpoint_capacity ? 1 : 0;
+    sums[0][threadIdx.x] = steps;
+    longest_of[threadIdx.x] = longest;
+    __syncthreads();
+    const auto scan = [&](int64_t (&values)[256]) {
+      int64_t running = 0;
+      for (int i = 0; i < static_cast<int>(blockDim.x); ++i) {
+        const int64_t value = values[i];
+        values[i] = running;
+        running += value;
+      }
+      return running;
+    };
+    int64_t all_steps = 0;
+    if (threadIdx.x == 0) {
+      longest = 0;
+      for (int i = 0; i < static_cast<int>(blockDim.x); ++i) longest = max(longest, longest_of[i]);
+      all_steps = scan(sums[0]);
+      step_prefix[S] = all_steps;
+      const int forced = pieces.forced_gradient_rows;
+      plan[0] = forced != 0 ? max(forced, 0)
+          : piece_rows_for(all_steps * H, longest, pieces.gradient_waves, kPieceRowsMin, kPieceAlign);
+      plan[1] = piece_rows_for(all_steps * H, longest, pieces.stats_waves, kPieceRowsMin, kChunk);
+    }
+    __syncthreads();
+    const int gradient_rows = plan[0], stats_rows = plan[1];
+    int64_t items[2] = {0, 0};
+    for (int s = first; s < last; ++s) {
+      items[0] += pieces_of_sequence(seq_len[s], gradient_rows) * H;
+      items[1] += pieces_of_sequence(seq_len[s], stats_rows) * H;
+    }
+    sums[1][threadIdx.x] = items[0];
+    sums[2][threadIdx.x] = items[1];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int64_t gradient_items = scan(sums[1]);
+      const int64_t stats_items = scan(sums[2]);
+      pieces.gradient_prefix[S] = static_cast<int32_t>(gradient_items);
+      pieces.stats_prefix[S] = static_cast<int32_t>(stats_items);
+      header[kHeaderGradientPieces] = gradient_rows;
+      header[kHeaderGradientPieces + 1] = static_cast<int32_t>(gradient_items);
+      header[kHeaderStatsPieces] = stats_items > pieces.stats_items_most ? 0 : stats_rows;
+      header[kHeaderStatsPieces + 1] = static_cast<int32_t>(stats_items);
+      header[3] = checkpoint_slots(all_steps * H, static_cast<int64_t>(block_prefix[S]) * H) <=
+                          checkpoint_capacity ? 1 : 0;
+    }
+    __syncthreads();
+    steps = sums[0][threadIdx.x];
+    items[0] = sums[1][threadIdx.x];
+    items[1] = sums[2][threadIdx.x];
+    for (int s = first; s < last; ++s) {
+      step_prefix[s] = steps;
+      pieces.gradient_prefix[s] = static_cast<int32_t>(items[0]);
+      pieces.stats_prefix[s] = static_cast<int32_t>(items[1]);
+      steps += band_steps_total(seq_len[s]);
+      items[0] += pieces_of_sequence(seq_len[s], gradient_rows) * H;
+      items[1] += pieces_of_sequence(seq_len[s], stats_rows) * H;
+    }
   }
   __syncthreads();
   int running = partial[threadIdx.x];
@@ -1032,14 +1102,8 @@ __global__ __launch_bounds__(256) void finalize_row_records_kernel(float4* __res
                                                                    float null_logit) {
   const int64_t index = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (index >= rows) return;
-  const float4 row = stats[index];
-  const float denominator = row.y + fast_exp2((null_logit - row.x) * kLog2e);
-  uint4 record;
-  record.x = 0u;
-  record.y = __float_as_uint(fmaf(row.x, kLog2e, row.w) + __log2f(denominator));
-  record.z = __float_as_uint(row.z / denominator);
-  record.w = 0u;
-  reinterpret_cast<uint4*>(stats)[index] = record;
+  const RowRecord record = row_record<true>(stats[index], null_logit);
+  reinterpret_cast<uint4*>(stats)[index] = make_uint4(0u, record.shift, record.expected, 0u);
 }
 
 // SIMDs of the current device (the persistent gradient kernel keeps as many waves resident
@@ -1081,38 +1145,52 @@ std::atomic<int> g_gradient_block_waves{0};  // 0: by shape
 std::atomic<int> g_gradient_piece_rows{0};
 
 // How the bands of the gradient kernel are cut into pieces (vjp_gradients_kernel): only with
-// single-wave blocks and when there are fewer than two bands per resident wave, so that the
-// longest band no longer sets the kernel's time.  A piece is at least four windows long (the
-// W - 1 rows below it are walked a second time) and a whole number of staged segments.
+// single-wave blocks, and only where whole bands would leave resident waves idle (a band is
+// as long as its diagonal, so the kernel would last as long as its longest one).  A piece is a
+// whole number of staged segments; piece_rows_for says how long.
 struct PiecePlan {
   int piece_rows;   // 0: whole bands
   int max_pieces;   // work items per band
 };
 
-PiecePlan plan_band_pieces(int64_t units, int longest, int W, int64_t resident_waves, int segment) {
+// rows of all bands of the problem; of a packed batch the most there can be (one sequence)
+int64_t band_rows_at_most(const Layout& L) {
+  return L.varlen ? static_cast<int64_t>(L.H) * band_steps_total(L.N)
+                  : static_cast<int64_t>(L.B) * L.H * band_steps_total(L.T);
+}
+
+PiecePlan plan_band_pieces(const Layout& L, int64_t resident_waves) {
   PiecePlan plan{0, 1};
-  const auto whole_segments = [&](int64_t rows) {
-    return static_cast<int>((std::max<int64_t>(rows, 2 * segment) + segment - 1) / segment * segment);
-  };
+  const int longest = L.varlen ? L.N : L.T;
+  const int64_t units = static_cast<int64_t>(L.slots) * L.H;
   int rows = 0;
   const int forced_rows = g_gradient_piece_rows.load(std::memory_order_relaxed);
   if (forced_rows > 0) {
-    rows = whole_segments(forced_rows);
+    rows = (std::max(forced_rows, 2 * kPieceAlign) + kPieceAlign - 1) / kPieceAlign * kPieceAlign;
+    if (longest - 1 <= rows) rows = 0;
   } else if (forced_rows == 0 && g_gradient_block_waves.load(std::memory_order_relaxed) != 2 &&
-             units > 0 &&
              units < 2 * resident_waves) {
-    const int64_t pieces_wanted = (2 * resident_waves + units - 1) / units;
-    rows = std::max(whole_segments(4 * static_cast<int64_t>(W)),
-                    whole_segments((longest - 1 + pieces_wanted - 1) / pieces_wanted));
+    // (a packed batch is cut on the device, by its actual lengths; here it counts as equal
+    // sequences)
+    const int64_t rows_in_all =
+        L.varlen ? static_cast<int64_t>(L.H) * L.S * band_steps_total(L.N / std::max(L.S, 1))
+                 : band_rows_at_most(L);
+    rows = piece_rows_for(rows_in_all, longest, resident_waves, kPieceRowsMin, kPieceAlign);
   }
-  if (rows <= 0 || longest - 1 <= rows) return plan;
-  const int64_t pieces = (static_cast<int64_t>(longest) - 1 + rows - 1) / rows;
-  if (units * pieces > INT32_MAX) return plan;
+  const int pieces = pieces_of_band(rows, longest);
+  if (rows <= 0 || pieces < 2 || units * pieces > INT32_MAX) return plan;
   plan.piece_rows = rows;
-  plan.max_pieces = static_cast<int>(pieces);
+  plan.max_pieces = pieces;
   return plan;
 }
 
+// waves of the row-statistics kernel that run at a time (four per SIMD at almost every width)
+int64_t resident_stats_waves() { return 4 * static_cast<int64_t>(device_simds()); }
+
+// Up to this many rows per resident wave the gradient pass runs as its three-term form alone,
+// which serves every input: below it the launch that returns at once would cost more than
+// the third term.
+constexpr int kSingleFormRows = 64;
 
 // How the gradient kernel is launched for a tile shape: waves per block, whether row tiles
 // are queued between the bands of a block, and the LDS of a block.
@@ -1389,7 +1467,9 @@ struct VjpWorkspace {
       value_bits, block_scratch, total;
   size_t sums_query, sums_key, sums_value;  // head-major accumulators (rows of <= 8 floats)
   bool symbols_by_head, values_by_head;
-  size_t checkpoints;
+  size_t checkpoints, chunk_decay;
+  int64_t stats_items_most;     // work items the row-statistics grid of a packed batch has room for
+  size_t gradient_prefix, stats_prefix;
   int64_t checkpoint_capacity;  // chunk records that fit in the workspace (0: none kept)
   int record_floats;
   int resident_blocks;
@@ -1408,6 +1488,8 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
   w.seq_len = cursor; cursor += align_up(sizeof(int32_t) * s);
   w.block_prefix = cursor; cursor += align_up(sizeof(int32_t) * (s + 1));
   w.step_prefix = cursor; cursor += align_up(sizeof(int64_t) * (s + 1));
+  w.gradient_prefix = cursor; cursor += align_up(sizeof(int32_t) * (s + 1));
+  w.stats_prefix = cursor; cursor += align_up(sizeof(int32_t) * (s + 1));
   const size_t rows = static_cast<size_t>(v.symbol_rows);
   const int slice_width = std::min(v.L.Dv, kValueSlice);
   const int dvp = padded_value_width(slice_width);
@@ -1443,6 +1525,8 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
     w.checkpoint_capacity = v.L.varlen ? std::min(wanted, budget) : (wanted <= budget ? wanted : 0);
     cursor += align_up(sizeof(float) * w.record_floats *
                        static_cast<size_t>(w.checkpoint_capacity));
+    w.chunk_decay = cursor;
+    cursor += align_up(sizeof(uint16_t) * static_cast<size_t>(w.checkpoint_capacity));
   }
   const int longest = v.L.varlen ? v.L.N : v.L.T;
   w.ring_rows = std::min(v.L.W, longest) + 1;
@@ -1469,9 +1553,16 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
   const int64_t units = static_cast<int64_t>(v.L.slots) * v.L.H;
   // resident waves of the gradient kernel (an even number: its blocks hold one or two waves)
   const int64_t resident_cap = resident_gradient_waves((dvp + 15) / 16, v.L.D > 16 ? 2 : 1);
-  const PiecePlan pieces = plan_band_pieces(units, longest, v.L.W, resident_cap, segment_rows);
-  w.resident_blocks = static_cast<int>(
-      std::min<int64_t>((units * pieces.max_pieces + 1) & ~int64_t(1), resident_cap));
+  // a piece per kPieceRowsMin rows or per resident wave's share, whichever is fewer, and one
+  // more per band (the last piece of a band is a short one)
+  w.stats_items_most =
+      2 * units + std::min(band_rows_at_most(v.L) / kPieceRowsMin, 2 * resident_stats_waves());
+  // (work items at most: whole bands, or pieces of at least kPieceRowsMin rows)
+  const PiecePlan pieces = plan_band_pieces(v.L, resident_cap);
+  const int64_t items = pieces.max_pieces > 1 || v.L.varlen
+      ? units + band_rows_at_most(v.L) / kPieceRowsMin : units;
+  w.resident_blocks =
+      static_cast<int>(std::min<int64_t>((items + 1) & ~int64_t(1), resident_cap));
   // keep the scratch pool below 2 GiB by running fewer resident blocks for huge windows
   const int64_t budget_floats = (int64_t(1) << 31) / 4;
   while (w.resident_blocks > 64 &&
@@ -1497,7 +1588,8 @@ unsigned blocks_for(int64_t items, int threads) {
 int launch_prepare_sequences(const rosa_problem* p, Layout& L, void* workspace, size_t seq_start,
                              size_t seq_len, size_t block_prefix, size_t header,
                              hipStream_t stream, int64_t* step_prefix = nullptr,
-                             int64_t checkpoint_capacity = 0) {
+                             int64_t checkpoint_capacity = 0,
+                             PieceLimits pieces = PieceLimits{}) {
   if (!L.varlen) return 0;
   L.seq_start = at<int32_t>(workspace, seq_start);
   L.seq_len = at<int32_t>(workspace, seq_len);
@@ -1506,7 +1598,7 @@ int launch_prepare_sequences(const rosa_problem* p, Layout& L, void* workspace, 
   hipLaunchKernelGGL(prepare_sequences_kernel, dim3(1), dim3(256), 0, stream, p->cu_seqlens, L.S,
                      L.N, at<int32_t>(workspace, seq_start), at<int32_t>(workspace, seq_len),
                      at<int32_t>(workspace, block_prefix), step_prefix, L.H, checkpoint_capacity,
-                     at<int32_t>(workspace, header));
+                     at<int32_t>(workspace, header), pieces);
   return 0;
 }
 
@@ -1685,37 +1777,48 @@ int launch_vjp_passes(int nvw, int dvp, int symbol_tiles, bool dropout, const Vj
     stage_end(kStageRowMax, stream);
     if (status != 0) return status;
   }
-  stage_begin(kStageRowStats, stream);
-  status = launch_band_kernel(row_kernels[vjp_kernel_slot_row_stats(varlen, dropout)], units,
-                              kWave, row_stats_dynamic_lds(P.grad_pitch), stream, Q);
-  if (status != 0) return status;
-  {
-    const int64_t rows = static_cast<int64_t>(P.L.N) * P.L.H;
-    hipLaunchKernelGGL(finalize_row_records_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0,
-                       stream, P.stats, rows, P.null_logit);
-  }
-  stage_end(kStageRowStats, stream);
-  const int segment = gradient_segment(dvp);
   const GradientBlockPlan plan = plan_gradient_blocks(dvp, P.L.D, nvw, P.grad_pitch, P.total_units);
   Q.wave_lds_floats = static_cast<int>(plan.wave_floats);
   Q.exchange_tile_floats = static_cast<int>(plan.tile_floats);
   Q.row_queue = plan.row_queue ? 1 : 0;
   Q.piece_rows = 0;
-  Q.max_pieces = 1;
+  const int64_t resident = resident_gradient_waves((dvp + 15) / 16, symbol_tiles);
   if (plan.waves == 1) {
-    const PiecePlan pieces = plan_band_pieces(
-        P.total_units, P.L.varlen ? P.L.N : P.L.T, P.L.W,
-        resident_gradient_waves((dvp + 15) / 16, symbol_tiles), segment);
+    const PiecePlan pieces = plan_band_pieces(P.L, resident);
     Q.piece_rows = pieces.piece_rows;
-    Q.max_pieces = pieces.max_pieces;
-    Q.total_units = P.total_units * pieces.max_pieces;
+    if (!varlen && Q.piece_rows > 0) {
+      Q.items = static_cast<int>(pieces_of_sequence(P.L.T, Q.piece_rows) * P.L.B * P.L.H);
+    }
   }
+  Q.gradient_pieces = Q.piece_rows > 0 ? 1 : 0;
+  stage_begin(kStageRowStats, stream);
+  {
+    int64_t blocks = varlen ? w.stats_items_most : units;
+    if (!varlen) {
+      Q.stats_piece_rows = piece_rows_for(band_rows_at_most(P.L), P.L.T, resident_stats_waves(),
+                                          kPieceRowsMin, kChunk);
+      if (Q.stats_piece_rows > 0) {
+        blocks = pieces_of_sequence(P.L.T, Q.stats_piece_rows) * P.L.B * P.L.H;
+      }
+    }
+    status = launch_band_kernel(row_kernels[vjp_kernel_slot_row_stats(varlen, dropout)],
+                                static_cast<unsigned>(blocks), kWave,
+                                row_stats_dynamic_lds(P.grad_pitch), stream, Q);
+    if (status != 0) return status;
+  }
+  if (Q.gradient_pieces == 0) {
+    const int64_t rows = static_cast<int64_t>(P.L.N) * P.L.H;
+    hipLaunchKernelGGL(finalize_row_records_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0,
+                       stream, P.stats, rows, P.null_logit);
+  }
+  stage_end(kStageRowStats, stream);
   const unsigned blocks = static_cast<unsigned>(std::max(1, w.resident_blocks / plan.waves));
   const int form = plan.waves == 2 ? kGradientFormTwoWaves
                                    : Q.piece_rows > 0 ? kGradientFormPieces : kGradientFormOneWave;
   stage_begin(kStageGradients, stream);
   // both forms of the kernel (see its TERMS): the one that does not apply returns at once
-  for (int terms = 2; terms <= 3 && status == 0; ++terms) {
+  Q.single_form = band_rows_at_most(P.L) <= kSingleFormRows * resident ? 1 : 0;
+  for (int terms = Q.single_form ? 3 : 2; terms <= 3 && status == 0; ++terms) {
     status = launch_band_kernel(kernels[vjp_kernel_slot_gradients(varlen, dropout, form, terms)],
                                 blocks, kWave * plan.waves, plan.lds_bytes, stream, Q);
   }
@@ -1739,8 +1842,18 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
             float* grad_key, float* grad_value, void* workspace, hipStream_t stream) {
   Layout L = view.L;
   const VjpWorkspace w = carve_vjp(view, dropout_p > 0.0f);
-  launch_prepare_sequences(p, L, workspace, w.seq_start, w.seq_len, w.block_prefix, w.header,
-                           stream, at<int64_t>(workspace, w.step_prefix), w.checkpoint_capacity);
+  {
+    const int dvp = padded_value_width(std::min(L.Dv, kValueSlice));
+    const int64_t resident = resident_gradient_waves((dvp + 15) / 16, L.D > 16 ? 2 : 1);
+    const int forced = g_gradient_piece_rows.load(std::memory_order_relaxed);
+    const PieceLimits limits{resident, resident_stats_waves(),
+                             forced > 0 ? plan_band_pieces(L, resident).piece_rows : forced,
+                             w.stats_items_most, at<int32_t>(workspace, w.gradient_prefix),
+                             at<int32_t>(workspace, w.stats_prefix)};
+    launch_prepare_sequences(p, L, workspace, w.seq_start, w.seq_len, w.block_prefix, w.header,
+                             stream, at<int64_t>(workspace, w.step_prefix), w.checkpoint_capacity,
+                             limits);
+  }
   // Value widths above 64 are processed in slices of 64 dimensions, one full backward per
   // slice: the route weights do not depend on the values, dV of a slice needs only that
   // slice, and dQ / dK are linear in the utilities, i.e. they are the sum over the slices.
@@ -1871,6 +1984,9 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
     P.block_scratch_floats = w.block_scratch_floats;
     P.segment_group = w.segment_group;
     P.ring_rows = w.ring_rows;
+    P.chunk_decay = at<uint16_t>(workspace, w.chunk_decay);
+    P.gradient_prefix = at<int32_t>(workspace, w.gradient_prefix);
+    P.stats_prefix = at<int32_t>(workspace, w.stats_prefix);
     P.total_units = L.slots * L.H;
     const bool dropout = dropout_p > 0.0f;
 
@@ -2969,9 +3085,7 @@ int rosa_hip_gradient_piece_plan(const rosa_problem* problem, int* piece_rows, i
       dvp, view.L.D, value_words(slice_width), grad_term_pitch(view.grad_terms, dvp), units);
   PiecePlan plan{0, 1};
   if (blocks.waves == 1) {
-    plan = plan_band_pieces(units, view.L.varlen ? view.L.N : view.L.T, view.L.W,
-                            resident_gradient_waves((dvp + 15) / 16, symbol_tiles),
-                            gradient_segment(dvp));
+    plan = plan_band_pieces(view.L, resident_gradient_waves((dvp + 15) / 16, symbol_tiles));
   }
   if (piece_rows != nullptr) *piece_rows = plan.piece_rows;
   if (pieces != nullptr) *pieces = plan.max_pieces;

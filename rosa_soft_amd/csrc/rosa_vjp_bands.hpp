@@ -52,9 +52,24 @@ struct VjpParams {
   int wave_lds_floats;          // LDS floats each wave of a gradient block owns
   int exchange_tile_floats;     // LDS floats of an accumulator tile passed between waves
   int row_queue;                // row tiles travel from band to band through LDS (two-wave blocks)
-  int piece_rows;               // rows of a piece of a band in the gradient pass (0: whole bands)
-  int max_pieces;               // work items per band: pieces of the longest possible band
+  // Bands are cut into pieces that different waves walk (0 rows: whole bands), `items` work items
+  // in all.  A packed batch takes these from the header (words 5 .. 8), where
+  // prepare_sequences_kernel has put them once it knew the lengths.
+  int piece_rows, items;        // of the gradient pass
+  int stats_piece_rows;         // of the row-statistics pass (items: its grid)
+  const int32_t* gradient_prefix;  // packed: pieces before each sequence
+  const int32_t* stats_prefix;
+  int gradient_pieces;          // the gradient pass runs in pieces: it reads chunk_decay
+  int single_form;              // only the three-term form of the gradient kernel is launched
+  uint16_t* chunk_decay;        // per chunk record: fewest mismatching bits any diagonal of the band
+                                // meets in the chunk's 16 rows
 };
+
+// header words that hold the piece plan of a packed batch
+constexpr int kHeaderGradientPieces = 5;  // rows, then work items in all
+constexpr int kHeaderStatsPieces = 7;
+constexpr int kPieceRowsMin = 32;   // rows of a piece at least
+constexpr int kPieceAlign = 32;     // pieces of the gradient pass are whole staged segments
 
 // Terms of the bfloat16 expansion of a float: x = t0 + t1 + t2 exactly (each term is the
 // bfloat16 nearest to what the terms before it leave), so that products with x can run on
@@ -94,6 +109,7 @@ struct BandView {
   const uint16_t* grad_rows;  // [t][grad_pitch] bfloat16 terms
   float4* stats;           // [t]
   float* checkpoints;      // chunk records of this band, or NULL
+  uint16_t* chunk_decay;   // with them: fewest mismatches of a diagonal, one entry per chunk
   int record_floats;
   int len;
   int diag0;               // first diagonal of the band
@@ -118,14 +134,31 @@ __device__ __forceinline__ void load_sliding(Band<NVW>& band, const BandView& vi
 //   4 exponent shift of the row    5 expected dropped utility
 //   6,7 unused
 // In the row-statistics pass the shift is that of the raw weight; in the gradient
-// pass the row records are final and the shift includes log2 of the denominator,
+// pass the sums of the row are complete and the shift includes log2 of the denominator,
 // so that exp2 gives the route probability directly.
 constexpr int kRowWords = 8;
-enum RowDetail { kRowSymbols = 0, kRowStats = 1, kRowFull = 2 };
+enum RowDetail { kRowSymbols = 0, kRowStats = 1, kRowSums = 2, kRowFinished = 3 };
+
+// What the gradient pass needs of a row, from the sums the row-statistics pass has left: the
+// exponent shift including log2 of the denominator and the expected dropped utility.  Whole
+// bands read it from finalize_row_records_kernel, a launch of its own between the two passes;
+// pieces, which small problems run as, form it where a row is staged (that launch cost them
+// 5 us of a step of 100; every band doing it again cost large problems 2 % of the pass).
+struct RowRecord {
+  uint32_t shift, expected;
+};
+
+template <bool FROM_SUMS>
+__device__ __forceinline__ RowRecord row_record(const float4& sums, float null_logit) {
+  if constexpr (!FROM_SUMS) return RowRecord{__float_as_uint(sums.y), __float_as_uint(sums.z)};
+  const float denominator = sums.y + fast_exp2((null_logit - sums.x) * kLog2e);
+  return RowRecord{__float_as_uint(fmaf(sums.x, kLog2e, sums.w) + __log2f(denominator)),
+                   __float_as_uint(sums.z / denominator)};
+}
 
 template <int NVW, int DETAIL>
 __device__ __forceinline__ void stage_rows(const BandView& view, int first, int count, int lane,
-                                           uint32_t* rows, int W) {
+                                           uint32_t* rows, int W, float null_logit = 0.0f) {
   for (int index = lane; index < count; index += kWave) {
     const int i = min(first + index, view.steps - 1);  // rows past the band's end repeat the last
     const int t = view.diag0 + 1 + i;
@@ -140,10 +173,10 @@ __device__ __forceinline__ void stage_rows(const BandView& view, int first, int 
     if constexpr (DETAIL == kRowStats) {
       const float4 row = view.stats[t];
       dst[1] = make_uint4(__float_as_uint(fmaf(row.x, kLog2e, row.w)), 0u, 0u, 0u);
-    } else if constexpr (DETAIL == kRowFull) {
-      const uint4 record = reinterpret_cast<const uint4*>(view.stats)[t];  // finalised
+    } else if constexpr (DETAIL == kRowSums || DETAIL == kRowFinished) {
+      const RowRecord record = row_record<DETAIL == kRowSums>(view.stats[t], null_logit);
       // the replay order of the gradient pass (staged_symbols_replay_order)
-      dst[0] = make_uint4(symbols.x, symbols.z, record.y, record.z);
+      dst[0] = make_uint4(symbols.x, symbols.z, record.shift, record.expected);
       dst[1] = make_uint4(symbols.y, symbols.w, 0u, 0u);
     }
   }
@@ -186,6 +219,7 @@ struct StepOut {
   float gate;     // local match gate of this pair
   float overflow; // product of the W+1 gates ending here (0 while the window is not full)
   float evidence; // S(t, a)
+  int mismatches; // bits in which the pair's symbols differ
   bool active;    // a >= 1
   int a;
 };
@@ -243,6 +277,7 @@ __device__ __forceinline__ StepOut forward_step(Band<NVW>& band, const RowSymbol
     return out;
   }
   const int mismatches = __popc(symbols.query ^ band.key_word);
+  out.mismatches = mismatches;
   const auto window_decay = [&]() {
     return BIASED ? decay_of_biased_count(band.window, gate_log2)
                   : fast_exp2(-gate_log2 * static_cast<float>(band.window));
@@ -298,6 +333,55 @@ __device__ __forceinline__ void sweep_rows(Band<NVW>& band, const uint32_t* rows
     for (int r = 0; r < count; ++r) {
       forward_step<NVW, false>(band, symbols_of(r), first + r, lane, W, gate_log2);
     }
+  }
+}
+
+// State of the band's diagonals in front of row `row` of a piece: the evidence is a sum over
+// the last W gates and the window a sum over the last W + 1, so a sweep over that many rows
+// from an empty state gives both (the overflow term matters from the last of them on only).
+// A quarter of the work of the rows that follow, and without LDS: 64 rows' words are held a
+// register each and handed out by lane number.
+template <int NVW>
+__device__ __forceinline__ void enter_piece(Band<NVW>& band, const BandView& view, int row, int lane,
+                                            int W, float gate_log2) {
+  band.evidence = 0.0f;
+  band.window = 0;
+  int first = row - W - 1;
+  // (where the sweep would meet rows in which some lane has no pair it starts with the band)
+  const bool whole = first < kWave;
+  if (whole) first = 0;
+  load_sliding<NVW>(band, view, first, lane, W);
+  for (int base = first; base < row; base += kWave) {
+    const int i = min(base + lane, row - 1);
+    const uint32_t query = view.q[view.diag0 + 1 + i];
+    const uint32_t key = view.k[i];
+    const int t_old = view.diag0 + i - W;
+    const uint32_t old_query = whole && t_old >= 0 ? view.q[t_old] : 0u;
+    const uint32_t old_key = whole && i - W - 1 >= 0 ? view.k[i - W - 1] : 0u;
+    const int count = min(kWave, row - base);
+    if (whole) {
+      for (int r = 0; r < count; ++r) {
+        const RowSymbols symbols{static_cast<uint32_t>(__builtin_amdgcn_readlane(query, r)),
+                                 static_cast<uint32_t>(__builtin_amdgcn_readlane(old_query, r)),
+                                 static_cast<uint32_t>(__builtin_amdgcn_readlane(key, r)),
+                                 static_cast<uint32_t>(__builtin_amdgcn_readlane(old_key, r))};
+        forward_step<NVW>(band, symbols, base + r, lane, W, gate_log2);
+      }
+    } else {
+      for (int r = 0; r < count; ++r) {
+        band.key_word = dpp_wave_shr1(static_cast<uint32_t>(__builtin_amdgcn_readlane(key, r)),
+                                      band.key_word);
+        const uint32_t differing =
+            static_cast<uint32_t>(__builtin_amdgcn_readlane(query, r)) ^ band.key_word;
+        const float gate = decay_of_biased_count(biased_popc(differing), gate_log2);
+        band.window = static_cast<int>(popc_plus(differing, static_cast<uint32_t>(band.window)));
+        band.evidence = fmaf(gate, band.evidence, gate);
+      }
+    }
+  }
+  if (!whole) {
+    band.evidence -= fast_exp2(-gate_log2 * static_cast<float>(band.window));
+    load_sliding<NVW>(band, view, row, lane, W);  // (the sweep has slid the key words only)
   }
 }
 
@@ -504,7 +588,7 @@ __device__ __forceinline__ void utility_tiles_staged(const uint16_t* grad_tile, 
   }
 }
 
-template <int NVW, bool VARLEN>
+template <int NVW, bool VARLEN, bool SCALAR = false>
 __device__ __forceinline__ bool make_view(const VjpParams& P, const Unit& u, BandView& view,
                                           int& value_head) {
   view.len = u.len;
@@ -524,8 +608,8 @@ __device__ __forceinline__ bool make_view(const VjpParams& P, const Unit& u, Ban
   int64_t steps_before, bands_before;
   const int blocks = (u.len + 63) >> 6;
   if constexpr (VARLEN) {
-    steps_before = P.L.step_prefix[u.seq] * P.L.H + u.head * band_steps_total(u.len);
-    bands_before = static_cast<int64_t>(P.L.block_prefix[u.seq]) * P.L.H + u.head * blocks;
+    steps_before = table_value<SCALAR>(P.L.step_prefix[u.seq]) * P.L.H + u.head * band_steps_total(u.len);
+    bands_before = static_cast<int64_t>(table_value<SCALAR>(P.L.block_prefix[u.seq])) * P.L.H + u.head * blocks;
   } else {
     const int64_t sequence_head = static_cast<int64_t>(u.seq) * P.L.H + u.head;
     steps_before = sequence_head * band_steps_total(u.len);
@@ -534,9 +618,12 @@ __device__ __forceinline__ bool make_view(const VjpParams& P, const Unit& u, Ban
   steps_before += band_steps_before(u.len, u.block);
   bands_before += u.block;
   view.checkpoints = nullptr;
+  view.chunk_decay = nullptr;
   view.record_floats = P.record_floats;
-  if (P.checkpoints != nullptr && (!VARLEN || P.header[3] != 0)) {
-    view.checkpoints = P.checkpoints + ((steps_before >> 4) + bands_before) * P.record_floats;
+  if (P.checkpoints != nullptr && (!VARLEN || table_value<SCALAR>(P.header[3]) != 0)) {
+    const int64_t slot = (steps_before >> 4) + bands_before;
+    view.checkpoints = P.checkpoints + slot * P.record_floats;
+    view.chunk_decay = P.chunk_decay + slot;
   }
   return true;
 }
@@ -648,11 +735,26 @@ void vjp_row_stats_kernel(VjpParams P) {
   constexpr int kWeightRows = kChunk / 2;
   __shared__ __attribute__((aligned(16))) float weights[kWeightRows * kWeightPitch];
   float* const discard = weights;
-  const Unit u = decode_unit<VARLEN>(P.L, blockIdx.x);
+  // (the host sizes the grid of a packed batch before it knows the lengths: blocks beyond the
+  // items it turns out to have return at once)
+  const int piece_rows = VARLEN ? table_value<true>(P.header[kHeaderStatsPieces]) : P.stats_piece_rows;
+  int piece = 0;
+  Unit u;
+  if (piece_rows > 0) {
+    if (VARLEN && static_cast<int>(blockIdx.x) >= P.header[kHeaderStatsPieces + 1]) return;
+    u = decode_piece<VARLEN>(P.L, P.stats_prefix, piece_rows, blockIdx.x, piece);
+  } else {
+    if (VARLEN && static_cast<int>(blockIdx.x) >= P.total_units) return;
+    u = decode_unit<VARLEN>(P.L, blockIdx.x);
+  }
   if (!u.valid) return;
   BandView view;
   int hv;
   if (!make_view<NVW, VARLEN>(P, u, view, hv)) return;
+  // rows [row_begin, row_end) of the band are this work item's
+  const int row_begin = piece * piece_rows;
+  if (row_begin >= view.steps) return;
+  const int row_end = piece_rows > 0 ? min(view.steps, row_begin + piece_rows) : view.steps;
   const int lane = threadIdx.x;
   const int W = P.L.W;
   DropoutKey key;
@@ -667,11 +769,10 @@ void vjp_row_stats_kernel(VjpParams P) {
   }
   const float logit_gain = in_vector_register(P.logit_gain);
   Band<NVW> band;
-  band.evidence = 0.0f;
-  band.window = kCountBias;  // forward_step<..., BIASED>
-  load_sliding<NVW>(band, view, 0, lane, W);
+  enter_piece<NVW>(band, view, row_begin, lane, W, P.gate_log2);
+  band.window += kCountBias;  // forward_step<..., BIASED>
   const bool needs_utility = (P.gradient_mask & (ROSA_GRAD_QUERY | ROSA_GRAD_KEY)) != 0;
-  uint32_t route_hash = route_hash_of(-lane);
+  uint32_t route_hash = route_hash_of(row_begin - lane);
   const int last_step = view.steps - 1;
   // without symbol gradients no utilities are computed and the tile stays zero
   for (int index = lane; index < kChunk * kUtilityPitch; index += kWave) utilities[index] = 0.0f;
@@ -760,6 +861,7 @@ void vjp_row_stats_kernel(VjpParams P) {
   int pending_window = 0;
   uint32_t pending_kept = 0u;
   int pending_first = -1, pending_rows = 0;
+  int pending_decay = 0;
   const auto flush_outputs = [&]() {
     if (pending_first < 0) return;
     // lanes 0..3 of every 16-lane group write the four rows of their group
@@ -774,6 +876,9 @@ void vjp_row_stats_kernel(VjpParams P) {
       float* slot =
           view.checkpoints + static_cast<int64_t>(pending_first / kChunk) * view.record_floats;
       reinterpret_cast<uint16_t*>(slot + kWave)[lane] = static_cast<uint16_t>(pending_window);
+      if (P.gradient_pieces != 0 && lane == 63) {
+        view.chunk_decay[pending_first / kChunk] = static_cast<uint16_t>(pending_decay);
+      }
       if constexpr (DROPOUT) {
         // the gradient pass reads the decisions back instead of hashing again
         reinterpret_cast<uint16_t*>(slot + kCheckpointFloats)[lane] =
@@ -782,9 +887,9 @@ void vjp_row_stats_kernel(VjpParams P) {
     }
     pending_first = -1;
   };
-  issue_block_loads(0);
-  for (int first = 0; first < view.steps; first += kBlockRows) {
-    const int count = min(kBlockRows, view.steps - first);
+  issue_block_loads(row_begin);
+  for (int first = row_begin; first < row_end; first += kBlockRows) {
+    const int count = min(kBlockRows, row_end - first);
     wave_lds_fence();
     if (lane < kBlockRows) {
       uint4* row_words = reinterpret_cast<uint4*>(rows + lane * kRowWords);
@@ -808,7 +913,7 @@ void vjp_row_stats_kernel(VjpParams P) {
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (first + kBlockRows < view.steps) issue_block_loads(first + kBlockRows);
+    if (first + kBlockRows < row_end) issue_block_loads(first + kBlockRows);
     __builtin_amdgcn_sched_barrier(0);
     for (int local = 0; local < count; local += kChunk) {
       const int rows_here = min(kChunk, count - local);
@@ -830,6 +935,7 @@ void vjp_row_stats_kernel(VjpParams P) {
         wave_lds_fence();
       }
       uint32_t kept_bits = 0u;  // bit r: this lane's pair of row r is kept
+      uint32_t entering = 0u;   // mismatching bits of this lane's pairs of the chunk
       v4f first_weight_sums;    // of rows 0 .. 7
       // compiled twice: once every lane is past its window fill no masking is needed
       auto run_chunk = [&](auto steady_tag, auto quiet_tag) {
@@ -839,7 +945,7 @@ void vjp_row_stats_kernel(VjpParams P) {
         // move a float32 result) and the window counts are only kept up to date: the
         // entering and the leaving mismatches are summed and applied after the chunk.
         constexpr bool QUIET = decltype(quiet_tag)::value;
-        uint32_t entering = 0u, leaving = 0u;
+        uint32_t leaving = 0u;
         // quiet chunks carry 1 + S: one fused multiply-add per row, and the root below
         // needs no addition (the weight only sees S through sqrt(1 + S) anyway)
         float one_plus_evidence = 1.0f + band.evidence;
@@ -957,6 +1063,7 @@ void vjp_row_stats_kernel(VjpParams P) {
             s.active = true;
           } else {
             s = forward_step<NVW, STEADY, false, true>(band, symbols, i, lane, W, P.gate_log2);
+            entering += static_cast<uint32_t>(s.mismatches);
             peak_overflow = fmaxf(peak_overflow, s.overflow);
           }
           // (outside quiet chunks the root is formed exactly as the gradient pass forms it:
@@ -1028,6 +1135,12 @@ void vjp_row_stats_kernel(VjpParams P) {
       // (random symbols of eight bits never reach it).  Header word 4; every writer writes 1.
       const bool long_match = __ballot(band.evidence >= kLongMatchEvidence) != 0ull;
       if ((noisy || long_match) && lane == 0) P.work_counter[3] = 1;
+      // (a chunk of the band's first rows, where lanes have no pair yet, or with rows beyond the
+      // band's end counts for nothing)
+      if (P.gradient_pieces != 0) {
+        pending_decay = chunk_first >= kWave && rows_here == kChunk
+                            ? wave_min_lane63(min(entering, 0xffffu)) : 0;
+      }
       pending_window = min(window_before, kRecordWindowMax) | (noisy ? 0x8000 : 0);
       pending_kept = kept_bits;
       pending_first = chunk_first;
@@ -1094,6 +1207,7 @@ constexpr int gradient_waves(int value_tiles, int symbol_tiles, bool pieces = fa
 // rows staged in LDS per segment of the gradient kernel (a multiple of kChunk): with 32 a
 // single-wave block of the narrowest tile needs 11.4 KB, which leaves room for three per SIMD
 constexpr int gradient_segment(int /*dvp*/) { return 32; }
+static_assert(kPieceAlign % gradient_segment(8) == 0, "pieces are whole staged segments");
 
 // Waves per block of the gradient kernel.  The waves of a block own neighbouring bands of
 // one (sequence, head) and walk them in step: at the same band-local step every band
@@ -1169,7 +1283,7 @@ void vjp_gradients_kernel(VjpParams P) {
   static_assert(NW == 1 || NW == 2, "blocks of one or two waves");
   static_assert(TERMS == 2 || TERMS == 3, "two or three terms per gate adjoint");
   static_assert(!PIECES || NW == 1, "pieces of bands are walked by single-wave blocks");
-  if ((P.header[4] != 0) != (TERMS == 3)) return;
+  if (P.single_form == 0 && (P.header[4] != 0) != (TERMS == 3)) return;
   constexpr int VT = (DVP + 15) / 16;   // value-dimension MFMA tiles
   constexpr bool kFetchAhead = true;  // row words and operands are fetched ahead of their use
   constexpr int SEG = gradient_segment(DVP);  // rows staged in LDS at a time
@@ -1255,51 +1369,82 @@ void vjp_gradients_kernel(VjpParams P) {
   fill_sign_table(sign_table, lane);
   wave_lds_fence();
 
+  // The first item of a block is its number; later ones come from the work counter, which
+  // starts at zero for item gridDim.x.  Pulls are atomics on one address, 40 ns each whoever
+  // makes them: with one per block in front of the first item and one behind the last, 2 048
+  // blocks spent 170 us of a short launch waiting for each other.  Where the grid has a block
+  // for every item there are none at all.
   int pulls = 0;
   for (;;) {
-    int unit_index = 0;
-    if constexpr (NW == 1) {
-      if (lane == 0) unit_index = atomicAdd(P.work_counter, 1);
-    } else {
-      // one pull per block; the two slots alternate, so that a wave that is still reading
-      // the previous index is not overtaken by the next pull
-      if (threadIdx.x == 0) shared_unit[pulls & 1] = atomicAdd(P.work_counter, 1);
-      block_barrier();
-      unit_index = shared_unit[pulls & 1];
-      ++pulls;
+    // (read again for every item: nothing of the plan stays in a register across one)
+    const int piece_rows =
+        PIECES ? (VARLEN ? table_value<true>(P.header[kHeaderGradientPieces]) : P.piece_rows) : 0;
+    const int total_items =
+        PIECES && piece_rows > 0 ? (VARLEN ? table_value<true>(P.header[kHeaderGradientPieces + 1])
+                                           : P.items)
+                                 : P.total_units;
+    int unit_index = static_cast<int>(blockIdx.x);
+    if (pulls > 0) {
+      const int grid = static_cast<int>(gridDim.x);
+      if (total_items <= grid) break;
+      if constexpr (NW == 1) {
+        if (lane == 0) unit_index = grid + atomicAdd(P.work_counter, 1);
+      } else {
+        // one pull per block; the two slots alternate, so that a wave that is still reading
+        // the previous index is not overtaken by the next pull
+        if (threadIdx.x == 0) shared_unit[pulls & 1] = grid + atomicAdd(P.work_counter, 1);
+        block_barrier();
+        unit_index = shared_unit[pulls & 1];
+      }
     }
+    ++pulls;
     unit_index = __builtin_amdgcn_readfirstlane(unit_index);
-    if (unit_index >= P.total_units) break;
+    if (unit_index >= total_items) break;
     // The unit names the first band of the block's group of NW neighbouring bands (the
     // longest of them); wave w takes band w of the group.  Everything that decides how often
     // the block meets at a barrier derives from the first band, which all waves know.
-    // With long bands and few of them a band is cut into pieces of `piece_rows` rows that
-    // different waves take (work item = band * max_pieces + piece): the kernel would otherwise
+    // With few bands per resident wave a band is cut into pieces of `piece_rows` rows that
+    // different waves take (decode_piece numbers them): the kernel would otherwise
     // last as long as its longest band.  The gate adjoints have a finite horizon (a row's
     // adjoint depends on the route adjoints of the W - 1 rows below it only), so a piece
-    // starts its reverse walk that many rows below its last row, with an empty carry and an
-    // empty window sum, and takes only the recurrences from those rows; its forward state
+    // starts its reverse walk at most that many rows below its last row, with an empty carry and
+    // an empty window sum, and takes only the recurrences from those rows; its forward state
     // comes from the chunk records (or the forward sweeps) like that of a whole band.
-    const int piece = PIECES ? unit_index % P.max_pieces : 0;
-    const Unit lead = decode_unit<VARLEN>(P.L, PIECES ? unit_index / P.max_pieces : unit_index);
+    int piece = 0;
+    const Unit lead = PIECES && piece_rows > 0
+        ? decode_piece<VARLEN>(P.L, P.gradient_prefix, piece_rows, unit_index, piece)
+        : decode_unit<VARLEN, NW == 1>(P.L, unit_index);
+    const int band_rows = lead.len - 1 - lead.block * kWave;
     if (!lead.valid) continue;
     if (NW > 1 && lead.block % NW != 0) continue;
-    const int band_rows = lead.len - 1 - lead.block * kWave;
     if (band_rows <= 0) continue;
     Unit u = lead;
     u.block += wave;
     BandView view;
     int hv;
-    const bool have_band = make_view<NVW, VARLEN>(P, u, view, hv);
+    const bool have_band = make_view<NVW, VARLEN, NW == 1>(P, u, view, hv);
     // rows [row_begin, row_end) are this work item's; the walk starts at row my_steps - 1
     int row_begin = 0, row_end = have_band ? view.steps : 0;
     int my_steps = row_end;  // a wave without a band only keeps step
     if constexpr (PIECES) {
-      row_begin = piece * P.piece_rows;
-      if (row_begin >= view.steps) continue;
-      row_end = min(view.steps, row_begin + P.piece_rows);
-      const int halo = (P.gradient_mask & (ROSA_GRAD_QUERY | ROSA_GRAD_KEY)) != 0
-          ? (P.L.W - 1 + kChunk - 1) / kChunk * kChunk : 0;
+      row_begin = piece * piece_rows;
+      row_end = piece_rows > 0 ? min(view.steps, row_begin + piece_rows) : view.steps;
+      int halo = 0;
+      if (want_qk) {
+        // At most the W - 1 rows of the horizon, and no more chunks than it takes for the gates
+        // of every diagonal to multiply to nothing: the carry that crosses them, and every
+        // overflow term whose window holds them, is then below `tail_threshold` of its value.
+        // Random symbols need one or two chunks, whatever the window.
+        const int most = (P.L.W - 1 + kChunk - 1) / kChunk;
+        const float enough = -__log2f(P.tail_threshold) / P.gate_log2;
+        float met = 0.0f;
+        int chunks = 0;
+        while (chunks < most && met < enough && row_end + kChunk * chunks < view.steps) {
+          if (view.chunk_decay != nullptr) met += view.chunk_decay[row_end / kChunk + chunks];
+          ++chunks;
+        }
+        halo = kChunk * chunks;
+      }
       my_steps = min(view.steps, row_end + halo);
     }
     const int lead_steps = PIECES ? my_steps : band_rows;
@@ -1521,9 +1666,8 @@ void vjp_gradients_kernel(VjpParams P) {
       }
       // one round trip brings in everything the segment needs
       wave_lds_fence();
-      // (all but the tightest variant: packed, Dv = 64, one wave per block has no registers
-      // for it and stages array by array, which took a quarter of the kernel at Dv = 64)
-      constexpr bool kHeavy = VT > 2 && VARLEN && NW == 1;
+      // (all but the tightest variant, which has no registers for it and stages array by array)
+      constexpr bool kHeavy = VT > 2 && VARLEN && DROPOUT && NW == 1 && TERMS == 3 && !PIECES;
       if constexpr (!kHeavy) {
         // Every global load of the segment is issued before the first of them is used, so
         // the segment costs one memory latency (two when the grad_output rows need the
@@ -1532,13 +1676,13 @@ void vjp_gradients_kernel(VjpParams P) {
         const int i = min(seg_first + lane, view.steps - 1);  // rows past the end repeat the last
         const int t = view.diag0 + 1 + i;
         uint4 symbols = make_uint4(0u, 0u, 0u, 0u);
-        uint4 record = make_uint4(0u, 0u, 0u, 0u);
+        float4 sums = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (row_lane) {
           symbols.x = view.q[t];
           symbols.y = (t - W - 1 >= 0) ? view.q[t - W - 1] : 0u;
           symbols.z = view.k[i];
           symbols.w = (i - W - 1 >= 0) ? view.k[i - W - 1] : 0u;
-          record = reinterpret_cast<const uint4*>(view.stats)[t];  // finalised
+          sums = view.stats[t];
         }
         constexpr int kKeyParts = (SEG + 2 * kWave - 1) / kWave;
         uint32_t key_in[kKeyParts], old_key_in[kKeyParts];
@@ -1552,7 +1696,8 @@ void vjp_gradients_kernel(VjpParams P) {
         const auto store_rows_and_keys = [&]() {
           if (row_lane) {
             uint4* row_words = reinterpret_cast<uint4*>(rows + lane * kRowWords);
-            row_words[0] = make_uint4(symbols.x, symbols.z, record.y, record.z);
+            const RowRecord record = row_record<PIECES>(sums, P.null_logit);
+            row_words[0] = make_uint4(symbols.x, symbols.z, record.shift, record.expected);
             row_words[1] = make_uint4(symbols.y, symbols.w, 0u, 0u);
             query_rows[lane] = seg_first + lane < view.steps ? symbols.x : 0u;
           }
@@ -1634,7 +1779,8 @@ void vjp_gradients_kernel(VjpParams P) {
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
-        stage_rows<NVW, kRowFull>(view, seg_first, SEG, lane, rows, W);
+        stage_rows<NVW, (PIECES ? kRowSums : kRowFinished)>(view, seg_first, SEG, lane, rows, W,
+                                                            P.null_logit);
         if (lane < SEG) {
           const int i = seg_first + lane;
           query_rows[lane] = i < view.steps ? view.q[view.diag0 + 1 + i] : 0u;

@@ -664,6 +664,38 @@ def test_bands_cut_into_pieces_match_oracle(cabi, c_oracle, records, B, T, H, D,
         assert_gradients_close(got, unsplit.cpu(), name + " against whole bands", slack)
 
 
+@pytest.mark.parametrize("lengths,W,p,pattern", [
+    ([33], 8, 0.0, "random"), ([34], 40, 0.1, "all_match"), ([65], 7, 0.0, "shifted"),
+    ([98], 16, 0.1, "random"), ([129], 200, 0.0, "periodic"), ([193], 31, 0.1, "shifted"),
+    ([577], 96, 0.0, "random"), ([33, 1, 0, 98, 2, 161, 64, 65], 24, 0.1, "shifted"),
+    ([640, 40, 257], 70, 0.0, "all_match"),
+])
+def test_small_problems_are_cut_by_shape_and_match_oracle(cabi, c_oracle, lengths, W, p, pattern):
+    """With fewer band rows than the chip has waves both passes walk pieces of bands (from 32
+    rows on): lengths around the edges of pieces, 16-row chunks and 64-diagonal bands, windows
+    shorter and longer than a piece, dense and packed."""
+
+    seed = 77 if p > 0 else None
+    total = sum(lengths)
+    query, key, value, grad_output = make_case(1, total, 2, 6, 1, 8, torch.float32, seed=total + W,
+                                               pattern=pattern)
+    offsets = None
+    if len(lengths) > 1:
+        query, key, value, grad_output = (t[0] for t in (query, key, value, grad_output))
+        offsets = [0] + [int(x) for x in np.cumsum(lengths)]
+    _, _, _, _, grads = run_device(cabi, query, key, value, grad_output, W, 1.0, p, 3.0, seed, 7,
+                                   offsets)
+    if offsets is None:
+        want = c_oracle.surrogate_vjp(query, key, value, grad_output, max_suffix_length=W,
+                                      dropout_p=p, seed=seed)
+    else:
+        want = c_oracle.varlen_surrogate_vjp(query, key, value, offsets, grad_output,
+                                             max_suffix_length=W, dropout_p=p, seed=seed)
+    slack = max(1.0, 2.4142 * ((1.0 + min(W, max(lengths))) ** 0.5 - 1.0) / 40.0)
+    for name, got, expected in zip(("grad_query", "grad_key", "grad_value"), grads, want):
+        assert_gradients_close(got, expected, name, slack)
+
+
 def test_atomic_rate_measurement_is_plausible_and_checks_its_arguments(cabi):
     """The measurement behind the gradient kernel's second bound: float atomics in the flush
     pattern (16 rows of a tile per step) run at some tens of G row segments per second on
