@@ -255,6 +255,15 @@ int rosa_hip_pack_symbols(int dtype, const void* logits, int64_t rows, int bits,
                           void* symbols, int symbol_bytes, void* stream);
 
 /*
+ * The inverse for the router's results: values[row, i] = +1 where bit i of symbols[row] is set,
+ * -1 where it is not, 0 in rows that matched nothing (matched_key_end[row] < 0).  `dtype` is the
+ * type of `values`, a contiguous [rows][bits] tensor.  Replaces unpack_sign_bits and the masking
+ * behind it in the reference's runtime front end (rosa_soft/runtime.py).
+ */
+int rosa_hip_unpack_symbols(int dtype, const uint8_t* symbols, const int64_t* matched_key_end,
+                            int64_t rows, int bits, void* values, void* stream);
+
+/*
  * Dense surrogate VJP.  Replaces surrogate_vjp_cuda (rosa_soft_kernels.cu:1923-2379)
  * and surrogate_vjp_varlen_cuda (:2382-2638).  Gradients are float32 in the
  * layout of the corresponding input and are fully overwritten; pass NULL for

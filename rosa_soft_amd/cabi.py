@@ -42,6 +42,7 @@ EXPORTED_SYMBOLS = (
     "rosa_hip_project_routed_bits",
     "rosa_hip_hard_forward_static",
     "rosa_hip_pack_symbols",
+    "rosa_hip_unpack_symbols",
     "rosa_hip_surrogate_vjp",
     "rosa_hip_router_update",
     "rosa_hip_router_workspace_bytes",
@@ -176,6 +177,9 @@ def load() -> ctypes.CDLL:
     library.rosa_hip_pack_symbols.argtypes = [
         ctypes.c_int, vp, ctypes.c_int64, ctypes.c_int, vp, ctypes.c_int, vp,
     ]
+    library.rosa_hip_unpack_symbols.restype = ctypes.c_int
+    library.rosa_hip_unpack_symbols.argtypes = [
+        ctypes.c_int, vp, vp, ctypes.c_int64, ctypes.c_int, vp, vp]
     library.rosa_hip_router_workspace_bytes.restype = ctypes.c_size_t
     library.rosa_hip_router_workspace_bytes.argtypes = [ctypes.POINTER(RosaRouterUpdate)]
     library.rosa_hip_router_update.restype = ctypes.c_int
@@ -484,6 +488,27 @@ def pack_symbols(logits: Tensor, symbol_dtype: torch.dtype = torch.uint8) -> Ten
     return symbols
 
 
+def unpack_symbols(symbols: Tensor, matched_key_end: Tensor, bits: int,
+                   dtype: torch.dtype) -> Tensor:
+    """The router's contiguous results as values of ``[..., bits]``: +1 or -1 per bit, 0 in rows
+    with ``matched_key_end < 0``.  ``dtype`` is float32, float16 or bfloat16.  One launch."""
+
+    if dtype not in _DTYPE_CODES:
+        raise ValueError("unpack_symbols supports float32, float16, and bfloat16")
+    if symbols.dtype != torch.uint8 or matched_key_end.dtype != torch.int64:
+        raise ValueError("symbols must be uint8 and positions int64")
+    assert symbols.is_cuda and symbols.shape == matched_key_end.shape
+    assert symbols.is_contiguous() and matched_key_end.is_contiguous()
+    with torch.cuda.device(symbols.device):
+        values = torch.empty((*symbols.shape, bits), dtype=dtype, device=symbols.device)
+        status = load().rosa_hip_unpack_symbols(
+            _DTYPE_CODES[dtype], _ptr(symbols), _ptr(matched_key_end), symbols.numel(), bits,
+            _ptr(values), _stream(symbols),
+        )
+    _check(status, "rosa_hip_unpack_symbols")
+    return values
+
+
 def hard_routes(
     query: Tensor,
     key: Tensor,
@@ -579,8 +604,10 @@ def vjp_workspace_bytes(query: Tensor, value: Tensor, max_suffix_length: int,
     return int(load().rosa_hip_vjp_workspace_bytes(ctypes.byref(problem), 7, 1.0, int(dropout)))
 
 
-def router_update(update: RosaRouterUpdate, device: torch.device) -> Optional[Tensor]:
-    """Enqueue one streaming-router update on the current stream of ``device``.
+def router_update(update: RosaRouterUpdate, device: torch.device,
+                  stream: Optional[torch.cuda.Stream] = None) -> Optional[Tensor]:
+    """Enqueue one streaming-router update on the current stream of ``device`` (``stream``: that
+    stream, where the caller has looked it up already).
 
     ``update.longest_total`` must be set.  Returns the workspace the update uses (or ``None``):
     the launches are stream-ordered, so the caller keeps it alive until they have run.
@@ -599,7 +626,8 @@ def router_update(update: RosaRouterUpdate, device: torch.device) -> Optional[Te
             update.workspace = workspace.data_ptr()
             update.workspace_bytes = size
         status = load().rosa_hip_router_update(
-            ctypes.byref(update), torch.cuda.current_stream(device).cuda_stream
+            ctypes.byref(update),
+            (stream if stream is not None else torch.cuda.current_stream(device)).cuda_stream
         )
     _check(status, "rosa_hip_router_update")
     return workspace

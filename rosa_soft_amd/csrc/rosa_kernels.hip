@@ -908,6 +908,52 @@ __global__ __launch_bounds__(256) void pack_rows_serial_kernel(const void* __res
   symbols[row] = static_cast<OUT>(symbol);
 }
 
+// What the router hands back as values: bit i of a symbol as +1 or -1, zeros where the row took
+// the null route (matched < 0).  WHOLE: symbols of eight bits to 16-byte aligned memory, a thread
+// per symbol and 16-byte stores; otherwise a thread per element.
+template <int DTYPE>
+__device__ __forceinline__ uint32_t unit_pattern(bool positive) {  // +1 or -1 in the type's bits
+  const uint32_t one = DTYPE == ROSA_DTYPE_F32 ? 0x3f800000u : DTYPE == ROSA_DTYPE_F16 ? 0x3c00u : 0x3f80u;
+  const uint32_t sign = DTYPE == ROSA_DTYPE_F32 ? 0x80000000u : 0x8000u;
+  return positive ? one : one | sign;
+}
+
+template <int DTYPE, bool WHOLE>
+__global__ __launch_bounds__(256) void unpack_symbols_kernel(const uint8_t* __restrict__ symbols,
+                                                             const int64_t* __restrict__ matched,
+                                                             int64_t items, int bits,
+                                                             void* __restrict__ values) {
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (item >= items) return;
+  if constexpr (WHOLE) {
+    const uint32_t symbol = symbols[item];
+    const bool routed = matched[item] >= 0;
+    constexpr int kPerWord = DTYPE == ROSA_DTYPE_F32 ? 1 : 2;
+    constexpr int kWords = 8 / kPerWord;
+    uint32_t words[kWords];
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) {
+      uint32_t word = unit_pattern<DTYPE>((symbol >> (kPerWord * w)) & 1u);
+      if constexpr (kPerWord == 2) word |= unit_pattern<DTYPE>((symbol >> (2 * w + 1)) & 1u) << 16;
+      words[w] = routed ? word : 0u;
+    }
+    uint4* target = static_cast<uint4*>(values) + item * (kWords / 4);
+#pragma unroll
+    for (int w = 0; w < kWords; w += 4)
+      target[w / 4] = make_uint4(words[w], words[w + 1], words[w + 2], words[w + 3]);
+  } else {
+    const int64_t row = item / bits;
+    const int bit = static_cast<int>(item - row * bits);
+    const uint32_t pattern =
+        matched[row] >= 0 ? unit_pattern<DTYPE>((symbols[row] >> bit) & 1u) : 0u;
+    if constexpr (DTYPE == ROSA_DTYPE_F32) {
+      static_cast<uint32_t*>(values)[item] = pattern;
+    } else {
+      static_cast<uint16_t*>(values)[item] = static_cast<uint16_t>(pattern);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // backward: preparation
 // ---------------------------------------------------------------------------
@@ -2049,9 +2095,13 @@ struct RouterUpdate {
   int blocks_per_run;            // blocks of the routing grid that share one (slot, head)
   // the index of the keys of every run, rebuilt by an update that uses it (NULL: none)
   int32_t* bucket_begin;         // [runs][2^qk_bits + 1]
-  uint2* bucket_routes;          // [runs][index_stride]: (route, key symbol before it), by bucket
+  void* bucket_routes;           // [runs][index_stride] RouterEntry::Word, by bucket
   uint8_t* run_scan;             // [runs]: 1 = the run is left to the scan
   uint8_t* left_over;            // [blocks of the routing grid]: 1 = left to the scan
+  // [runs][route_stride]: the routes of the update's rows, for router_emit_kernel (NULL: the
+  // routing kernel writes the results itself)
+  int32_t* routes;
+  int route_stride;
   int index_stride;
   int log_buckets;
   int budget_base;
@@ -2059,6 +2109,133 @@ struct RouterUpdate {
 
 __device__ __forceinline__ int router_chunk_begin(const RouterUpdate& U, int slot) {
   return U.chunk_offsets != nullptr ? U.chunk_offsets[slot] : slot * U.uniform_chunk;
+}
+
+// The (slot, head) and the block of 64 rows that a block of the routing grid takes: runs one
+// after the other, the latest rows (the longest walks) first, as in the training forward.  Blocks
+// go to the eight dies in turn, so with a multiple of eight runs all blocks of a run share a
+// die's cache and its copy of the run's index, and every compute unit gets row blocks of every
+// length.  Run by run (2 slots x 64 heads x 4096 tokens) the walk took 40 us.
+struct RouterBlock {
+  int run, row_block;
+};
+
+__device__ __forceinline__ RouterBlock router_block(const RouterUpdate& U) {
+  const unsigned runs = static_cast<unsigned>(U.S) * static_cast<unsigned>(U.H);
+  const unsigned from_last = blockIdx.x / runs;
+  return {static_cast<int>(blockIdx.x - from_last * runs),
+          U.blocks_per_run - 1 - static_cast<int>(from_last)};
+}
+
+// Chunks of 64 tokens or more: a block takes 64 tokens x 64 heads of one slot and turns them
+// through LDS.  Inputs are token-major and histories run-major; a thread per symbol wrote every
+// byte to a line of its own (8 slots x 4096 tokens x 64 heads: 31.8 us, bound by the partial
+// lines that leave the caches, now 6.3 us).
+constexpr int kRouterTileRows = 64;
+constexpr int kRouterTileHeads = 64;
+constexpr int kRouterTilePitch = kRouterTileHeads + 1;
+
+__global__ __launch_bounds__(256) void router_append_tile_kernel(RouterUpdate U, int row_tiles,
+                                                                 int head_tiles) {
+  __shared__ uint8_t tile[3][kRouterTileRows * kRouterTilePitch];
+  const int head_tile = static_cast<int>(blockIdx.x) % head_tiles;
+  const int slot_tile = static_cast<int>(blockIdx.x) / head_tiles;
+  const int row_tile = slot_tile % row_tiles;
+  const int slot = slot_tile / row_tiles;
+  const int chunk_begin = router_chunk_begin(U, slot);
+  const int first = row_tile * kRouterTileRows;
+  const int rows = min(kRouterTileRows, router_chunk_begin(U, slot + 1) - chunk_begin - first);
+  if (rows <= 0) return;
+  const int head0 = head_tile * kRouterTileHeads;
+  const int heads = min(kRouterTileHeads, U.H - head0);
+  const int payload_heads = min(kRouterTileHeads, U.Hp - head0);  // may be negative
+  const int64_t token = chunk_begin + first;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  // (past the tile's edges the last row or head is read again, so that no load waits for a
+  // branch and all of a thread's are in flight together)
+  constexpr int kParts = kRouterTileRows / 4;
+  uint8_t queries[kParts], keys[kParts], payloads[kParts];
+  const int head = head0 + min(lane, heads - 1);
+  const int payload_head = head0 + min(lane, payload_heads - 1);
+#pragma unroll
+  for (int part = 0; part < kParts; ++part) {
+    const int64_t row = token + min(wave + 4 * part, rows - 1);
+    queries[part] = U.query[row * U.H + head];
+    keys[part] = U.key[row * U.H + head];
+    payloads[part] = payload_heads > 0 ? U.payload[row * U.Hp + payload_head] : uint8_t(0);
+  }
+#pragma unroll
+  for (int part = 0; part < kParts; ++part) {
+    const int slot_of_tile = (wave + 4 * part) * kRouterTilePitch + lane;
+    tile[0][slot_of_tile] = queries[part] & U.qk_mask;
+    tile[1][slot_of_tile] = keys[part] & U.qk_mask;
+    tile[2][slot_of_tile] = payloads[part] & U.payload_mask;
+  }
+  __syncthreads();
+  const int position = U.history_lengths[slot] + first + lane;
+  if (lane >= rows) return;
+#pragma unroll 4
+  for (int h = wave; h < heads; h += 4) {
+    const int64_t run = (static_cast<int64_t>(slot) * U.H + head0 + h) * U.capacity + position;
+    U.query_history[run] = tile[0][lane * kRouterTilePitch + h];
+    U.key_history[run] = tile[1][lane * kRouterTilePitch + h];
+  }
+  for (int h = wave; h < payload_heads; h += 4) {
+    U.payload_history[(static_cast<int64_t>(slot) * U.Hp + head0 + h) * U.capacity + position] =
+        tile[2][lane * kRouterTilePitch + h];
+  }
+}
+
+// The results of an indexed update, from the routes its routing kernels have left run-major: a
+// block takes 32 tokens x 64 heads of one slot, reads the routes and the payloads they name
+// lane = row, and writes symbols and positions token-major in whole lines.  Written by the
+// routing kernels themselves, lane = row, every position was an eight-byte piece of a line of
+// its own, put together from up to 64 blocks (8 slots x 4096 tokens x 64 heads: 30 of the
+// candidate walk's 122 us, where this kernel takes 10).
+constexpr int kRouterEmitRows = 32;
+
+__global__ __launch_bounds__(256) void router_emit_kernel(RouterUpdate U, int row_tiles,
+                                                          int head_tiles) {
+  __shared__ int32_t route_tile[kRouterEmitRows * kRouterTilePitch];
+  __shared__ uint8_t symbol_tile[kRouterEmitRows * kRouterTilePitch];
+  const int head_tile = static_cast<int>(blockIdx.x) % head_tiles;
+  const int slot_tile = static_cast<int>(blockIdx.x) / head_tiles;
+  const int row_tile = slot_tile % row_tiles;
+  const int slot = slot_tile / row_tiles;
+  const int chunk_begin = router_chunk_begin(U, slot);
+  const int first = row_tile * kRouterEmitRows;
+  const int rows = min(kRouterEmitRows, router_chunk_begin(U, slot + 1) - chunk_begin - first);
+  if (rows <= 0) return;
+  const int head0 = head_tile * kRouterTileHeads;
+  const int heads = min(kRouterTileHeads, U.H - head0);
+  const int group = U.H / U.Hp;
+  const int row = threadIdx.x & (kRouterEmitRows - 1);
+  if (row < rows) {
+#pragma unroll 4
+    for (int h = threadIdx.x / kRouterEmitRows; h < heads; h += 256 / kRouterEmitRows) {
+      const int head = head0 + h;
+      const int route =
+          U.routes[(static_cast<int64_t>(slot) * U.H + head) * U.route_stride + first + row];
+      uint8_t symbol = 0;
+      if (route > 0) {
+        symbol = U.payload_history[(static_cast<int64_t>(slot) * U.Hp + head / group) * U.capacity +
+                                   route];
+      }
+      route_tile[row * kRouterTilePitch + h] = route;
+      symbol_tile[row * kRouterTilePitch + h] = symbol;
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  if (lane >= heads) return;
+#pragma unroll 4
+  for (int r = threadIdx.x >> 6; r < rows; r += 4) {
+    const int64_t index = static_cast<int64_t>(chunk_begin + first + r) * U.H + head0 + lane;
+    const int route = route_tile[r * kRouterTilePitch + lane];
+    U.matched_key_end[index] = route > 0 ? route - 1 : -1;
+    U.output[index] = symbol_tile[r * kRouterTilePitch + lane];
+  }
 }
 
 __global__ __launch_bounds__(256) void router_append_kernel(RouterUpdate U) {
@@ -2093,10 +2270,10 @@ __global__ __launch_bounds__(256) void router_append_kernel(RouterUpdate U) {
 __global__ __launch_bounds__(kWave) void router_route_kernel(RouterUpdate U) {
   // (behind router_candidates_kernel: only the row blocks that kernel has left over)
   if (U.left_over != nullptr && U.left_over[blockIdx.x] == 0) return;
-  // one-dimensional grid: (slot, head) run-major, so that slots * heads is not bounded by
-  // the 65535 blocks of the other grid dimensions
-  const int run = static_cast<int>(blockIdx.x / static_cast<unsigned>(U.blocks_per_run));
-  const int row_block = static_cast<int>(blockIdx.x - static_cast<unsigned>(run) * U.blocks_per_run);
+  // one-dimensional grid, so that slots * heads is not bounded by the 65535 blocks of the
+  // other grid dimensions
+  const RouterBlock block = router_block(U);
+  const int run = block.run, row_block = block.row_block;
   const int slot = run / U.H;
   const int head = run - slot * U.H;
   const int old_length = U.history_lengths[slot];
@@ -2118,6 +2295,10 @@ __global__ __launch_bounds__(kWave) void router_route_kernel(RouterUpdate U) {
              : scan_routes_wide(q, k, t0, new_length, U.W, lane, q_symbol);
   if (!row_ok) return;
   const int route = winner.run > 0 ? winner.route : 0;
+  if (U.routes != nullptr) {
+    U.routes[static_cast<int64_t>(run) * U.route_stride + (t - old_length)] = route;
+    return;
+  }
   const int64_t token = chunk_begin + (t - old_length);
   const int payload_head = head / (U.H / U.Hp);
   U.matched_key_end[token * U.H + head] = route > 0 ? route - 1 : -1;
@@ -2126,9 +2307,30 @@ __global__ __launch_bounds__(kWave) void router_route_kernel(RouterUpdate U) {
       : uint8_t(0);
 }
 
+// An entry of the index: the route and the key symbol before it (route 1 has none: a value no
+// symbol takes).  NARROW: histories below 2^23 tokens, where both fit one word.
+template <bool NARROW>
+struct RouterEntry {
+  using Word = std::conditional_t<NARROW, uint32_t, uint2>;
+  static __device__ __forceinline__ Word make(uint32_t route, uint32_t before) {
+    if constexpr (NARROW) return (route << 9) | before;
+    else return make_uint2(route, before);
+  }
+  static __device__ __forceinline__ uint32_t route(const Word& word) {
+    if constexpr (NARROW) return word >> 9;
+    else return word.x;
+  }
+  static __device__ __forceinline__ uint32_t before(const Word& word) {
+    if constexpr (NARROW) return word & 0x1ffu;
+    else return word.y;
+  }
+};
+constexpr int kRouterNarrowBelow = 1 << 23;
+
 // The index of the keys for the router (see index_keys_kernel): byte symbols, one bucket per
 // symbol, the whole history of a run indexed anew by every update that routes a long chunk.
-// An entry is the route and the key symbol before it; the key symbol itself is the bucket's.
+// The key symbol itself is the bucket's.
+template <bool NARROW>
 __global__ __launch_bounds__(kIndexThreads) void router_index_kernel(RouterUpdate U) {
   __shared__ int cursor[256];
   __shared__ int partial[256];
@@ -2172,23 +2374,24 @@ __global__ __launch_bounds__(kIndexThreads) void router_index_kernel(RouterUpdat
     U.run_scan[run] = largest > max(64, count / 16) ? 1 : 0;
   }
   __syncthreads();
-  uint2* routes = U.bucket_routes + static_cast<int64_t>(run) * U.index_stride;
+  using Entry = RouterEntry<NARROW>;
+  typename Entry::Word* routes = static_cast<typename Entry::Word*>(U.bucket_routes) +
+                                 static_cast<int64_t>(run) * U.index_stride;
   for (int p0 = 0; p0 < count; p0 += kIndexThreads) {  // ordered passes, as in index_keys_kernel
     const int p = p0 + thread;
     if (p < count) {
-      // (route 1 has no key before it: a value no symbol takes)
-      routes[atomicAdd(&cursor[k[p]], 1)] =
-          make_uint2(static_cast<uint32_t>(p + 1), p >= 1 ? static_cast<uint32_t>(k[p - 1]) : 0x100u);
+      routes[atomicAdd(&cursor[k[p]], 1)] = Entry::make(
+          static_cast<uint32_t>(p + 1), p >= 1 ? static_cast<uint32_t>(k[p - 1]) : 0x100u);
     }
     __syncthreads();
   }
 }
 
+template <bool NARROW>
 __global__ __launch_bounds__(kWave) void router_candidates_kernel(RouterUpdate U) {
-  const int run = static_cast<int>(blockIdx.x / static_cast<unsigned>(U.blocks_per_run));
-  const int row_block = static_cast<int>(blockIdx.x - static_cast<unsigned>(run) * U.blocks_per_run);
+  const RouterBlock block = router_block(U);
+  const int run = block.run, row_block = block.row_block;
   const int slot = run / U.H;
-  const int head = run - slot * U.H;
   const int lane = threadIdx.x;
   const int old_length = U.history_lengths[slot];
   const int chunk_begin = router_chunk_begin(U, slot);
@@ -2209,39 +2412,61 @@ __global__ __launch_bounds__(kWave) void router_candidates_kernel(RouterUpdate U
   const int32_t* begin = U.bucket_begin + static_cast<int64_t>(run) * (buckets + 1);
   int next = row_ok ? begin[q_symbol] : 0;
   const int end = row_ok ? begin[q_symbol + 1] : 0;
-  const uint2* routes = U.bucket_routes + static_cast<int64_t>(run) * U.index_stride;
+  using Entry = RouterEntry<NARROW>;
+  const typename Entry::Word* routes =
+      static_cast<const typename Entry::Word*>(U.bucket_routes) +
+      static_cast<int64_t>(run) * U.index_stride;
   const int budget = U.budget_base + t0 / 8;
   const int walk_budget = budget / 4;
   int spent = 0, walked = 0;  // wave-uniform
   uint64_t best = 0;          // (run << 32) | route
-  uint2 ahead = next < end ? routes[next] : make_uint2(0u, 0x100u);
-  while (__builtin_amdgcn_ballot_w64(next < end) != 0ull) {
-    const bool have = next < end;
-    const int a = static_cast<int>(ahead.x);
-    const uint32_t key_before = ahead.y;
-    ++next;
-    if (next < end) ahead = routes[next];
-    if (have && ((a - 1) & ~(kIndexThreads - 1)) >= t) next = end;
-    const bool candidate = have && a <= t;
-    const int limit = min(U.W, a);
-    int length = candidate ? 1 : 0;
-    bool walking = candidate && limit >= 2 && key_before == q_before;
-    if (walking) length = 2;
-    walking = walking && length < limit;
-    while (walked <= walk_budget && __builtin_amdgcn_ballot_w64(walking) != 0ull) {
-      ++walked;
-      if (walking) {
-        if (q[t - length] == k[a - 1 - length]) {
-          ++length;
-          walking = length < limit;
-        } else {
-          walking = false;
+  // A lane walks its bucket through dependent round trips to the index, so it keeps the next
+  // four entries in flight (one at a time: 32 us where this takes 18, 2 slots x 64 heads x
+  // 4096 tokens; 8 slots 122 us before the routes went out run-major, now 57).
+  constexpr int kAhead = 4;
+  typename Entry::Word ahead[kAhead];
+  const auto fetch = [&](int first) {
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      ahead[j] = first + j < end ? routes[first + j] : Entry::make(0u, 0x100u);
+    }
+  };
+  bool beyond = false;  // the entries left belong to passes that begin beyond this row
+  fetch(next);
+  while (__builtin_amdgcn_ballot_w64(next < end && !beyond) != 0ull) {
+    typename Entry::Word entries[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) entries[j] = ahead[j];
+    const int first = next;
+    next += kAhead;
+    fetch(next);
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const bool have = first + j < end && !beyond;
+      const int a = static_cast<int>(Entry::route(entries[j]));
+      if (have && ((a - 1) & ~(kIndexThreads - 1)) >= t) beyond = true;
+      const bool candidate = have && a <= t;
+      const int limit = min(U.W, a);
+      int length = candidate ? 1 : 0;
+      bool walking = candidate && limit >= 2 && Entry::before(entries[j]) == q_before;
+      if (walking) length = 2;
+      walking = walking && length < limit;
+      while (walked <= walk_budget && __builtin_amdgcn_ballot_w64(walking) != 0ull) {
+        ++walked;
+        if (walking) {
+          if (q[t - length] == k[a - 1 - length]) {
+            ++length;
+            walking = length < limit;
+          } else {
+            walking = false;
+          }
         }
       }
+      const uint64_t found = (static_cast<uint64_t>(length) << 32) | static_cast<uint32_t>(a);
+      if (candidate) best = max(best, found);
     }
-    const uint64_t found = (static_cast<uint64_t>(length) << 32) | static_cast<uint32_t>(a);
-    if (candidate) best = max(best, found);
-    if (++spent > budget || walked > walk_budget) {
+    spent += kAhead;
+    if (spent > budget || walked > walk_budget) {
       if (lane == 0) U.left_over[blockIdx.x] = 1;
       return;
     }
@@ -2249,12 +2474,7 @@ __global__ __launch_bounds__(kWave) void router_candidates_kernel(RouterUpdate U
   if (lane == 0) U.left_over[blockIdx.x] = 0;
   if (!row_ok) return;
   const int route = (best >> 32) > 0 ? static_cast<int>(best & 0xffffffffu) : 0;
-  const int64_t token = chunk_begin + (t - old_length);
-  const int payload_head = head / (U.H / U.Hp);
-  U.matched_key_end[token * U.H + head] = route > 0 ? route - 1 : -1;
-  U.output[token * U.H + head] = route > 0
-      ? U.payload_history[(static_cast<int64_t>(slot) * U.Hp + payload_head) * U.capacity + route]
-      : uint8_t(0);
+  U.routes[static_cast<int64_t>(run) * U.route_stride + (t - old_length)] = route;
 }
 
 // Few new rows per slot (decoding): one wave per (slot, head, new row); the lanes share the
@@ -2312,13 +2532,20 @@ __global__ __launch_bounds__(256) void router_advance_kernel(RouterUpdate U) {
 // wave can append its row, route it and leave the new length without waiting for any other
 // wave (three launches otherwise: append, route, advance, each waiting for the one before).
 // Symbols at positions from the old length on are the chunk's own and are read from the
-// update's inputs, so that no wave depends on another's append.
-__global__ __launch_bounds__(kWave) void router_decode_step_kernel(RouterUpdate U) {
+// update's inputs, so that no block depends on another's append.
+//
+// Bound by memory round trips one behind the other.  Four waves per row take sixteen stored keys
+// per thread with one load, a history of 4096 in one trip, and follow a match eight symbols at a
+// time: 8 slots x 64 heads at 4096 keys take 7.4 us where one wave reading bytes took 14.5 us.
+constexpr int kDecodeThreads = 256;
+
+__global__ __launch_bounds__(kDecodeThreads) void router_decode_step_kernel(RouterUpdate U) {
+  __shared__ unsigned long long best_of_wave[kDecodeThreads / kWave];
   const int run = static_cast<int>(blockIdx.x / static_cast<unsigned>(U.blocks_per_run));
   const int row = static_cast<int>(blockIdx.x - static_cast<unsigned>(run) * U.blocks_per_run);
   const int slot = run / U.H;
   const int head = run - slot * U.H;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x;  // of the block
   const int old_length = U.history_lengths[slot];
   const int chunk_begin = router_chunk_begin(U, slot);
   const int rows = router_chunk_begin(U, slot + 1) - chunk_begin;
@@ -2352,28 +2579,77 @@ __global__ __launch_bounds__(kWave) void router_decode_step_kernel(RouterUpdate 
   }
   const uint32_t q_symbol = q_at(t);
   unsigned long long best = 0ull;
-  constexpr int kAhead = 4;  // key symbols a lane has in flight
-  for (int a0 = 1 + lane; a0 <= t; a0 += kAhead * kWave) {
-    uint32_t keys[kAhead];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      const int a = a0 + j * kWave;
-      keys[j] = a <= t ? k_at(a - 1) : 0x100u;
+  // a key position whose symbol is the row's: how far the symbols before it agree as well
+  const auto extend = [&](int position) {
+    const int a = position + 1;
+    const int limit = min(U.W, a);
+    int length = 1;
+    while (length < limit) {
+      if (limit - length >= 8 && t - length < old_length) {  // eight symbols of both histories
+        unsigned long long queries, keys;
+        __builtin_memcpy(&queries, q_history + (t - length - 7), 8);
+        __builtin_memcpy(&keys, k_history + (a - 1 - length - 7), 8);
+        const unsigned long long differing = queries ^ keys;
+        if (differing == 0ull) {
+          length += 8;
+          continue;
+        }
+        length += __clzll(static_cast<long long>(differing)) >> 3;
+        break;
+      }
+      if (q_at(t - length) != k_at(a - 1 - length)) break;
+      ++length;
     }
+    best = max(best, (static_cast<unsigned long long>(length) << 32) | static_cast<uint32_t>(a));
+  };
+  // the stored keys, sixteen per thread and round trip
+  struct Piece {
+    uint32_t words[4];
+  };
+  const unsigned stored = static_cast<unsigned>(old_length);
+  const auto load_piece = [&](unsigned first) {
+    Piece piece = {};
+    if (first + 16 <= stored) {
+      __builtin_memcpy(piece.words, k_history + first, 16);
+    } else {
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      if (keys[j] != q_symbol) continue;
-      const int a = a0 + j * kWave;
-      const int limit = min(U.W, a);
-      int length = 1;
-      while (length < limit && q_at(t - length) == k_at(a - 1 - length)) ++length;
-      best = max(best, (static_cast<unsigned long long>(length) << 32) | static_cast<uint32_t>(a));
+      for (int j = 0; j < 16; ++j) {
+        if (first + j < stored)
+          piece.words[j / 4] |= static_cast<uint32_t>(k_history[first + j]) << (8 * (j % 4));
+      }
+    }
+    return piece;
+  };
+  constexpr unsigned kStride = 16 * kDecodeThreads;
+  unsigned first = 16 * static_cast<unsigned>(lane);
+  Piece ahead = load_piece(first);
+  for (; first < stored; first += kStride) {
+    const Piece piece = ahead;
+    ahead = load_piece(first + kStride);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t differing = piece.words[w] ^ (q_symbol * 0x01010101u);
+      // (a set top bit may also stand above a byte that is zero: looked at again below)
+      uint32_t equal = (differing - 0x01010101u) & ~differing & 0x80808080u;
+      while (equal != 0u) {
+        const int byte = __ffs(static_cast<int>(equal)) >> 3;
+        equal &= equal - 1u;
+        const unsigned position = first + 4 * w + (byte - 1);
+        if (((differing >> (8 * (byte - 1))) & 0xffu) == 0u && position < stored)
+          extend(static_cast<int>(position));
+      }
     }
   }
+  // the chunk's own keys before this row
+  if (lane < row && k_at(old_length + lane) == q_symbol) extend(old_length + lane);
 #pragma unroll
   for (int offset = 32; offset > 0; offset >>= 1) {
     best = max(best, static_cast<unsigned long long>(__shfl_xor(best, offset, kWave)));
   }
+  if ((lane & (kWave - 1)) == 0) best_of_wave[lane / kWave] = best;
+  __syncthreads();
+#pragma unroll
+  for (int wave = 0; wave < kDecodeThreads / kWave; ++wave) best = max(best, best_of_wave[wave]);
   if (lane != 0) return;
   const int route = (best >> 32) > 0 ? static_cast<int>(best & 0xffffffffull) : 0;
   const int64_t token = chunk_begin + row;
@@ -2651,11 +2927,25 @@ void launch_pack_rows(const void* logits, int64_t rows, int bits, void* symbols,
   }
 }
 
+template <int DTYPE>
+void launch_unpack_symbols(const uint8_t* symbols, const int64_t* matched, int64_t rows, int bits,
+                           void* values, hipStream_t stream) {
+  if (bits == 8 && (reinterpret_cast<uintptr_t>(values) & 15) == 0) {
+    hipLaunchKernelGGL((unpack_symbols_kernel<DTYPE, true>), dim3(blocks_for(rows, 256)), dim3(256),
+                       0, stream, symbols, matched, rows, bits, values);
+  } else {
+    hipLaunchKernelGGL((unpack_symbols_kernel<DTYPE, false>), dim3(blocks_for(rows * bits, 256)),
+                       dim3(256), 0, stream, symbols, matched, rows * bits, bits, values);
+  }
+}
+
 // The router's index of the keys in the caller's workspace: bucket offsets, routes by bucket,
-// one byte per run and one per block of the routing grid.
+// one byte per run and one per block of the routing grid, the routes of the update's rows.
 struct RouterWorkspace {
-  size_t bucket_begin, bucket_routes, run_scan, left_over, total;
+  size_t bucket_begin, bucket_routes, run_scan, left_over, routes, total;
   int blocks_per_run;
+  int route_stride;
+  bool narrow;  // one word per entry of the index
 };
 
 // Updates the index is used for: symbols of six bits or more (as in the training forward),
@@ -2673,10 +2963,14 @@ RouterWorkspace carve_router(const rosa_router_update& u) {
   w.blocks_per_run = (u.longest_chunk + kWave - 1) / kWave;
   size_t cursor = 0;
   w.bucket_begin = cursor; cursor += align_up(sizeof(int32_t) * runs * ((size_t(1) << u.qk_bits) + 1));
+  w.narrow = u.longest_total < kRouterNarrowBelow;
   w.bucket_routes = cursor;
-  cursor += align_up(sizeof(uint2) * runs * static_cast<size_t>(std::max(u.longest_total, 1)));
+  cursor += align_up((w.narrow ? sizeof(uint32_t) : sizeof(uint2)) * runs * static_cast<size_t>(std::max(u.longest_total, 1)));
   w.run_scan = cursor; cursor += align_up(runs);
   w.left_over = cursor; cursor += align_up(runs * static_cast<size_t>(std::max(w.blocks_per_run, 1)));
+  w.route_stride = std::max(w.blocks_per_run, 1) * kWave;
+  w.routes = cursor;
+  cursor += align_up(sizeof(int32_t) * runs * static_cast<size_t>(w.route_stride));
   w.total = cursor;
   return w;
 }
@@ -2833,6 +3127,29 @@ int rosa_hip_pack_symbols(int dtype, const void* logits, int64_t rows, int bits,
   return 0;
 }
 
+int rosa_hip_unpack_symbols(int dtype, const uint8_t* symbols, const int64_t* matched_key_end,
+                            int64_t rows, int bits, void* values, void* stream) {
+  if (dtype < ROSA_DTYPE_F32 || dtype > ROSA_DTYPE_BF16) return fail(1, "unsupported dtype");
+  if (bits < 1 || bits > 8) return fail(1, "unpack_symbols: symbol width must be in [1, 8]");
+  if (rows < 0 || rows > (int64_t{1} << 38)) return fail(1, "unpack_symbols: bad row count");
+  if (rows == 0) return 0;
+  if (!symbols || !matched_key_end || !values) return fail(2, "unpack_symbols: NULL pointer");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case ROSA_DTYPE_F32:
+      launch_unpack_symbols<ROSA_DTYPE_F32>(symbols, matched_key_end, rows, bits, values, s);
+      break;
+    case ROSA_DTYPE_F16:
+      launch_unpack_symbols<ROSA_DTYPE_F16>(symbols, matched_key_end, rows, bits, values, s);
+      break;
+    default:
+      launch_unpack_symbols<ROSA_DTYPE_BF16>(symbols, matched_key_end, rows, bits, values, s);
+  }
+  const hipError_t launch = hipGetLastError();
+  if (launch != hipSuccess) return fail_hip(launch, "unpack_symbols launch");
+  return 0;
+}
+
 int rosa_hip_hard_forward(const rosa_problem* problem, const void* query, const void* key,
                           const void* value, void* output, int32_t* packed_query,
                           int32_t* packed_key, int32_t* routes, void* workspace,
@@ -2929,18 +3246,22 @@ int rosa_hip_router_update(const rosa_router_update* update, void* stream) {
   U.tokens = u.tokens;
   U.blocks_per_run = 1;
   U.bucket_begin = nullptr; U.bucket_routes = nullptr; U.run_scan = nullptr; U.left_over = nullptr;
+  U.routes = nullptr; U.route_stride = 0;
   U.index_stride = 0; U.log_buckets = 0; U.budget_base = 0;
   const int index_mode = g_forward_index_mode.load(std::memory_order_relaxed);
-  bool indexed = false;
+  bool indexed = false, narrow = false;
   if (u.workspace != nullptr && index_mode != 1 && router_index_suits(u)) {
     if (u.longest_total > u.capacity)
       return fail(1, "router: longest_total exceeds the capacity of a run");
     const RouterWorkspace w = carve_router(u);
     if (u.workspace_bytes < w.total) return fail(3, "router: workspace too small");
     U.bucket_begin = at<int32_t>(u.workspace, w.bucket_begin);
-    U.bucket_routes = at<uint2>(u.workspace, w.bucket_routes);
+    U.bucket_routes = at<void>(u.workspace, w.bucket_routes);
+    narrow = w.narrow;
     U.run_scan = at<uint8_t>(u.workspace, w.run_scan);
     U.left_over = at<uint8_t>(u.workspace, w.left_over);
+    U.routes = at<int32_t>(u.workspace, w.routes);
+    U.route_stride = w.route_stride;
     U.index_stride = std::max(u.longest_total, 1);
     U.log_buckets = u.qk_bits;
     U.budget_base = index_mode == 2 ? -(1 << 30) : 64;
@@ -2955,10 +3276,26 @@ int rosa_hip_router_update(const rosa_router_update* update, void* stream) {
     U.blocks_per_run = u.longest_chunk;
     const int64_t blocks = runs * U.blocks_per_run;
     if (blocks > INT32_MAX) return fail(1, "router: slots * heads * row blocks must fit in int32");
-    hipLaunchKernelGGL(router_decode_step_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kWave),
-                       0, s, U);
+    hipLaunchKernelGGL(router_decode_step_kernel, dim3(static_cast<unsigned>(blocks)),
+                       dim3(kDecodeThreads), 0, s, U);
   } else {
-    hipLaunchKernelGGL(router_append_kernel, dim3(blocks_for(symbols, 256)), dim3(256), 0, s, U);
+    // Grids over (slot, tile of rows, tile of heads) exist where the longest chunk fills a tile
+    // of rows; shorter chunks (a tile would be mostly empty) take a thread per symbol.
+    const int head_tiles = (u.H + kRouterTileHeads - 1) / kRouterTileHeads;
+    const int64_t append_tiles = static_cast<int64_t>(u.S) * head_tiles *
+                                 ((u.longest_chunk + int64_t{kRouterTileRows} - 1) / kRouterTileRows);
+    const int64_t emit_tiles = static_cast<int64_t>(u.S) * head_tiles *
+                               ((u.longest_chunk + int64_t{kRouterEmitRows} - 1) / kRouterEmitRows);
+    if (indexed && emit_tiles > INT32_MAX)
+      return fail(1, "router: slots * heads * row blocks must fit in int32");
+    if (u.longest_chunk >= kRouterTileRows && append_tiles <= INT32_MAX) {
+      hipLaunchKernelGGL(router_append_tile_kernel, dim3(static_cast<unsigned>(append_tiles)),
+                         dim3(256), 0, s, U,
+                         static_cast<int>((u.longest_chunk + int64_t{kRouterTileRows} - 1) / kRouterTileRows),
+                         head_tiles);
+    } else {
+      hipLaunchKernelGGL(router_append_kernel, dim3(blocks_for(symbols, 256)), dim3(256), 0, s, U);
+    }
     if (u.longest_chunk > 0) {
       U.blocks_per_run = decode ? u.longest_chunk : (u.longest_chunk + kWave - 1) / kWave;
       const int64_t blocks = runs * U.blocks_per_run;
@@ -2968,13 +3305,19 @@ int rosa_hip_router_update(const rosa_router_update* update, void* stream) {
                            0, s, U);
       } else {
         if (indexed) {
-          hipLaunchKernelGGL(router_index_kernel, dim3(static_cast<unsigned>(runs)),
-                             dim3(kIndexThreads), 0, s, U);
-          hipLaunchKernelGGL(router_candidates_kernel, dim3(static_cast<unsigned>(blocks)),
-                             dim3(kWave), 0, s, U);
+          hipLaunchKernelGGL(narrow ? router_index_kernel<true> : router_index_kernel<false>,
+                             dim3(static_cast<unsigned>(runs)), dim3(kIndexThreads), 0, s, U);
+          hipLaunchKernelGGL(narrow ? router_candidates_kernel<true> : router_candidates_kernel<false>,
+                             dim3(static_cast<unsigned>(blocks)), dim3(kWave), 0, s, U);
         }
         hipLaunchKernelGGL(router_route_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kWave),
                            0, s, U);
+        if (indexed) {
+          hipLaunchKernelGGL(router_emit_kernel, dim3(static_cast<unsigned>(emit_tiles)), dim3(256),
+                             0, s, U,
+                             static_cast<int>((u.longest_chunk + int64_t{kRouterEmitRows} - 1) / kRouterEmitRows),
+                             head_tiles);
+        }
       }
     }
     hipLaunchKernelGGL(router_advance_kernel, dim3(blocks_for(u.S, 256)), dim3(256), 0, s, U);

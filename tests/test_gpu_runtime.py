@@ -419,6 +419,122 @@ def test_ragged_long_chunks_route_through_the_index_of_the_keys(rosa):
                 done[slot] += step[slot]
 
 
+@pytest.mark.parametrize("heads,payload_heads", [(70, 35), (9, 1), (64, 64), (130, 65)])
+def test_tiles_of_rows_and_heads_are_appended_and_emitted_whole(rosa, heads, payload_heads):
+    # chunks of 64 rows or more are turned in tiles of 64 x 64 symbols, indexed ones leave in
+    # tiles of 32 rows x 64 heads; the routing grid deals runs to the dies in groups of eight.
+    # Ragged chunks on both sides of the tile edges, more and fewer heads than a tile holds.
+    # Whole symbols and positions: exact, against the oracle.
+    bits, horizon = 6, 20
+    lengths = [[513, 64], [31, 577], [65, 1], [64, 33], [3, 63]]  # per update, per slot
+    totals = [sum(step[slot] for step in lengths) for slot in range(2)]
+    streams = []
+    for slot, total in enumerate(totals):
+        query = random_packed((1, total, heads), bits, 300 + slot)
+        key = random_packed((1, total, heads), bits, 310 + slot)
+        payload = random_packed((1, total, payload_heads), bits, 320 + slot)
+        streams.append((query, key, payload, expect_dense(query, key, payload, bits, bits, horizon)))
+    done = [0, 0]
+    with rosa.RosaRuntime(heads, payload_heads, bits, bits, horizon) as runtime:
+        for step in lengths:
+            rows = [slice(done[slot], done[slot] + step[slot]) for slot in range(2)]
+            parts = [torch.cat([s[i][0, rows[slot]] for slot, s in enumerate(streams)]).to(DEVICE)
+                     for i in range(3)]
+            output, ends = runtime.update_packed(
+                *parts, cu_seqlens=torch.tensor([0, step[0], sum(step)], dtype=torch.int32))
+            for part, got in enumerate((output, ends)):
+                want = torch.cat([s[3][part][0, rows[slot]] for slot, s in enumerate(streams)])
+                assert torch.equal(got.cpu(), want), (step, part)
+            done = [done[slot] + step[slot] for slot in range(2)]
+
+
+@pytest.mark.parametrize("prefill", [1, 7, 15, 16, 17, 63, 4094, 4096, 4100])
+@pytest.mark.parametrize("pattern", ["random", "period5", "binary"])
+def test_decoding_steps_read_every_piece_of_the_history(rosa, prefill, pattern):
+    # a decoding step reads stored keys sixteen at a time by 256 threads and follows matches
+    # eight symbols at a time: histories on both sides of those edges, matches shorter and longer
+    # than a stride, a window inside them, chunks of 1, 8 and 3 rows.  Exact, against all rows
+    # routed in one update by the scan over all routes.
+    from rosa_soft_amd import cabi
+
+    slots, heads, payload_heads, horizon = 2, 3, 3, 21
+    bits = 1 if pattern == "binary" else 8
+    steps = [prefill, 1, 8, 3, 1]
+    total = sum(steps)
+    query, key = (random_packed((slots, total, heads), bits, 400 + i) for i in range(2))
+    if pattern == "period5":
+        key = key[:, :5].repeat(1, total // 5 + 1, 1)[:, :total].contiguous()
+        query = torch.roll(key, 1, dims=1).contiguous()
+        query[1, 3::29] ^= 1
+    payload = random_packed((slots, total, payload_heads), 8, 402)
+    streams = [tensor.to(DEVICE) for tensor in (query, key, payload)]
+    cabi.set_forward_index("scan")
+    try:
+        with rosa.RosaRuntime(heads, payload_heads, bits, 8, horizon) as whole:
+            want = whole.update_packed(*streams)
+    finally:
+        cabi.set_forward_index(None)
+    done = 0
+    with rosa.RosaRuntime(heads, payload_heads, bits, 8, horizon) as runtime:
+        for rows in steps:
+            got = runtime.update_packed(*(tensor[:, done:done + rows] for tensor in streams))
+            for part in range(2):
+                assert torch.equal(got[part], want[part][:, done:done + rows]), (done, rows, part)
+            done += rows
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64])
+@pytest.mark.parametrize("bits", [1, 3, 8])
+def test_routed_symbols_unpack_to_signs_and_exact_zeros(rosa, bits, dtype):
+    # +1 and -1 per bit, zeros on the null route; odd row counts, whole and partial symbols
+    query, key = (random_packed((1, 77, 3), 2, 500 + i).to(DEVICE) for i in range(2))
+    payload = random_packed((1, 77, 3), bits, 502).to(DEVICE)
+    results = []
+    for packed in (True, False):
+        with rosa.RosaRuntime(3, 3, 2, bits, 4) as runtime:
+            results.append(runtime.update_packed(query, key, payload, return_packed=packed,
+                                                 output_dtype=dtype))
+    (symbols, ends), (values, _) = results
+    shifts = torch.arange(bits, device=DEVICE)
+    want = ((symbols.long().unsqueeze(-1) >> shifts) & 1) * 2 - 1
+    want = want * (ends >= 0).unsqueeze(-1)
+    assert values.dtype == dtype and values.shape == want.shape
+    assert bool((ends < 0).any()) and torch.equal(values, want.to(dtype))
+
+
+def test_index_entries_of_two_words_route_like_those_of_one(rosa):
+    # histories declared to reach 2^23 tokens keep the route and the key symbol before it in two
+    # words, shorter ones in one: the same update both ways, exact
+    from rosa_soft_amd import cabi
+
+    slots, heads, bits, horizon, tokens = 2, 3, 8, 17, 700
+    streams = [random_packed((slots, tokens, heads), bits, 600 + i).to(DEVICE) for i in range(3)]
+    streams[1][:, 400:600] = streams[1][:, 100:300]
+    streams[0][:, 401:600] = streams[1][:, 400:599]
+    results = []
+    for longest_total in (tokens, 2**23):
+        histories = [torch.zeros(slots, heads, longest_total, dtype=torch.uint8, device=DEVICE)
+                     for _ in range(3)]
+        lengths = torch.zeros(slots, dtype=torch.int32, device=DEVICE)
+        output = torch.empty(slots, tokens, heads, dtype=torch.uint8, device=DEVICE)
+        ends = torch.empty(slots, tokens, heads, dtype=torch.int64, device=DEVICE)
+        update = cabi.RosaRouterUpdate(
+            S=slots, H=heads, Hp=heads, W=horizon, qk_bits=bits, payload_bits=bits,
+            capacity=longest_total, tokens=slots * tokens, longest_chunk=tokens,
+            uniform_chunk=tokens, longest_total=longest_total)
+        update.history_lengths = lengths.data_ptr()
+        update.query_history, update.key_history, update.payload_history = (
+            h.data_ptr() for h in histories)
+        update.query, update.key, update.payload = (t.data_ptr() for t in streams)
+        update.output, update.matched_key_end = output.data_ptr(), ends.data_ptr()
+        workspace = cabi.router_update(update, torch.device(DEVICE))
+        torch.cuda.synchronize()
+        assert workspace is not None and lengths.tolist() == [tokens] * slots
+        results.append((output, ends))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert int((results[0][1][:, 401:600] >= 0).sum()) > 0
+
+
 # --------------------------------------------------------------------------- the reference's
 # interface tests (tests/test_runtime.py:344-1008) restated for the device runtime
 
