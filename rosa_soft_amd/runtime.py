@@ -101,7 +101,9 @@ def _slot_ids(sequence_ids, slot_count: int) -> Optional[Tuple[int, ...]]:
 
 
 def _flatten_packed(query: Tensor, key: Tensor, payload: Tensor, cu_seqlens: Optional[Tensor]):
-    """Token-major ``[total, H]`` views, host offsets, the output shape and the layout flag."""
+    """Contiguous token-major symbols (of either rank), the total of tokens, the tokens of every
+    slot, host offsets (None for the dense layout, where all slots bring the same number) and the
+    shape of the results without their head axis."""
 
     if any(tensor.dtype != torch.uint8 for tensor in (query, key, payload)):
         raise TypeError("packed RosaRuntime inputs must have dtype torch.uint8")
@@ -117,13 +119,8 @@ def _flatten_packed(query: Tensor, key: Tensor, payload: Tensor, cu_seqlens: Opt
         slots, tokens, _ = query.shape
         if slots < 1:
             raise ValueError("dense batch size must be >= 1")
-        offsets = [slot * tokens for slot in range(slots + 1)]
-        return (
-            query.reshape(slots * tokens, query.size(2)).contiguous(),
-            key.reshape(slots * tokens, key.size(2)).contiguous(),
-            payload.reshape(slots * tokens, payload.size(2)).contiguous(),
-            offsets, tuple(payload.shape), True,
-        )
+        return (query.contiguous(), key.contiguous(), payload.contiguous(), slots * tokens,
+                [tokens] * slots, None, (slots, tokens))
     if query.ndim != 2 or payload.ndim != 2:
         raise ValueError("varlen packed inputs must have shapes [total, H] and [total, H_v]")
     if query.size(0) != payload.size(0):
@@ -142,8 +139,9 @@ def _flatten_packed(query: Tensor, key: Tensor, payload: Tensor, cu_seqlens: Opt
         raise RuntimeError("cu_seqlens must be monotonic")
     if offsets[-1] != query.size(0):
         raise RuntimeError("query has wrong total token dimension")
-    return query.contiguous(), key.contiguous(), payload.contiguous(), offsets, \
-        tuple(payload.shape), False
+    return (query.contiguous(), key.contiguous(), payload.contiguous(), query.size(0),
+            [after - before for before, after in zip(offsets[:-1], offsets[1:])], offsets,
+            (query.size(0),))
 
 
 class _RuntimeWork:
@@ -252,6 +250,9 @@ class RosaRuntime:
         self._query_history: Optional[Tensor] = None    # [S, H, capacity] uint8
         self._key_history: Optional[Tensor] = None      # [S, H, capacity] uint8
         self._payload_history: Optional[Tensor] = None  # [S, Hp, capacity] uint8
+        # the library's description of an update, as far as updates share it; made anew when
+        # the histories it points to are
+        self._update: Optional[cabi.RosaRouterUpdate] = None
         self._last_update = None            # event recorded after the latest update's launches
         self._last_stream = None            # ... and the stream they went to
 
@@ -386,14 +387,14 @@ class RosaRuntime:
                         cu_seqlens: Optional[Tensor], *, stream, async_op: bool,
                         return_packed: bool, output_dtype: torch.dtype, sequence_ids,
                         caller_device: torch.device):
-        query, key, payload, offsets, output_shape, dense = _flatten_packed(
+        query, key, payload, tokens, chunks, offsets, lead = _flatten_packed(
             query_symbols, key_symbols, payload_symbols, cu_seqlens
         )
-        if query.size(1) != self.num_heads:
+        if query.size(-1) != self.num_heads:
             raise ValueError("packed query/key head count must equal num_heads")
-        if payload.size(1) != self.num_payload_heads:
+        if payload.size(-1) != self.num_payload_heads:
             raise ValueError("packed payload head count must equal num_payload_heads")
-        slot_count = len(offsets) - 1
+        slot_count = len(chunks)
         normalized_ids = _slot_ids(sequence_ids, slot_count)
         if stream is not None and caller_device.type != "cuda":
             raise ValueError("stream requires CUDA inputs")
@@ -420,18 +421,19 @@ class RosaRuntime:
             working_stream = torch.cuda.current_stream(self._device)
             if self._last_update is not None and working_stream != self._last_stream:
                 working_stream.wait_event(self._last_update)
-            output, ends = self._route(
-                query.to(self._device), key.to(self._device), payload.to(self._device), offsets
-            )
-            if dense:
-                output = output.reshape(output_shape[0], output_shape[1], self.num_heads)
-                ends = ends.reshape(output_shape[0], output_shape[1], self.num_heads)
+            if caller_device != self._device or query.device != self._device:
+                query, key, payload = (tensor.to(self._device) for tensor in (query, key, payload))
+            output, ends = self._route(query, key, payload, tokens, chunks, offsets, lead,
+                                       working_stream)
             if not return_packed:
-                unpacked = _unpack_sign_bits(output, self.payload_bits, output_dtype)
-                output = torch.where(
-                    ends.unsqueeze(-1) >= 0, unpacked,
-                    torch.zeros((), dtype=output_dtype, device=self._device),
-                )
+                if output_dtype in (torch.float32, torch.float16, torch.bfloat16):
+                    output = cabi.unpack_symbols(output, ends, self.payload_bits, output_dtype)
+                else:
+                    unpacked = _unpack_sign_bits(output, self.payload_bits, output_dtype)
+                    output = torch.where(
+                        ends.unsqueeze(-1) >= 0, unpacked,
+                        torch.zeros((), dtype=output_dtype, device=self._device),
+                    )
             # (one event, recorded anew by every update; an update on the stream of the one
             # before it is ordered by the stream itself)
             if self._last_update is None:
@@ -490,48 +492,59 @@ class RosaRuntime:
                 grown[..., : self._capacity] = old
             setattr(self, name, grown)
         self._capacity = capacity
+        self._update = None
 
-    def _route(self, query: Tensor, key: Tensor, payload: Tensor, offsets) -> Tuple[Tensor, Tensor]:
-        tokens = query.size(0)
-        output = torch.empty((tokens, self._num_heads), dtype=torch.uint8, device=self._device)
-        ends = torch.empty((tokens, self._num_heads), dtype=torch.int64, device=self._device)
+    def _route(self, query: Tensor, key: Tensor, payload: Tensor, tokens: int, chunks,
+               offsets, lead, stream) -> Tuple[Tensor, Tensor]:
+        shape = (*lead, self._num_heads)
+        output = torch.empty(shape, dtype=torch.uint8, device=self._device)
+        ends = torch.empty(shape, dtype=torch.int64, device=self._device)
         if tokens == 0:
             return output, ends
-        chunk_lengths = [after - before for before, after in zip(offsets[:-1], offsets[1:])]
-        self._grow(max(old + new for old, new in zip(self._lengths, chunk_lengths)))
+        lengths = [old + new for old, new in zip(self._lengths, chunks)]
+        longest_chunk, longest_total = max(chunks), max(lengths)
+        self._grow(longest_total)
         if self._device_lengths is None:
             # two arrays taking turns: an update reads one and writes the advanced lengths to the
-            # other, which makes a decoding step one launch
-            self._device_lengths = torch.tensor(self._lengths, dtype=torch.int32).to(self._device)
+            # other, which makes a decoding step one launch.  (A fresh runtime's are zeros, filled
+            # on the device: the copy of a host tensor waits for everything enqueued before it.)
+            if any(self._lengths):
+                self._device_lengths = torch.tensor(self._lengths, dtype=torch.int32).to(self._device)
+            else:
+                self._device_lengths = torch.zeros(len(chunks), dtype=torch.int32,
+                                                   device=self._device)
             self._device_lengths_next = torch.empty_like(self._device_lengths)
-        uniform = all(length == chunk_lengths[0] for length in chunk_lengths)
+        uniform = offsets is None or min(chunks) == longest_chunk
         tables = None if uniform else torch.tensor(offsets, dtype=torch.int32).to(self._device)
-        update = cabi.RosaRouterUpdate()
-        update.S, update.H, update.Hp = self._slot_count, self._num_heads, self._num_payload_heads
-        update.W = min(self._max_suffix_length, 2**31 - 1)
-        update.qk_bits, update.payload_bits = self._qk_bits, self._payload_bits
-        update.capacity = self._capacity
+        update = self._update
+        if update is None:  # what every update has in common until the histories grow
+            update = self._update = cabi.RosaRouterUpdate()
+            update.S, update.H, update.Hp = self._slot_count, self._num_heads, self._num_payload_heads
+            update.W = min(self._max_suffix_length, 2**31 - 1)
+            update.qk_bits, update.payload_bits = self._qk_bits, self._payload_bits
+            update.capacity = self._capacity
+            update.query_history = self._query_history.data_ptr()
+            update.key_history = self._key_history.data_ptr()
+            update.payload_history = self._payload_history.data_ptr()
         update.tokens = tokens
-        update.longest_chunk = max(chunk_lengths)
-        update.uniform_chunk = chunk_lengths[0] if uniform else 0
+        update.longest_chunk = longest_chunk
+        update.uniform_chunk = longest_chunk if uniform else 0
         update.chunk_offsets = None if uniform else tables.data_ptr()
         update.history_lengths = self._device_lengths.data_ptr()
         update.history_lengths_out = self._device_lengths_next.data_ptr()
-        update.query_history = self._query_history.data_ptr()
-        update.key_history = self._key_history.data_ptr()
-        update.payload_history = self._payload_history.data_ptr()
         update.query, update.key, update.payload = \
             query.data_ptr(), key.data_ptr(), payload.data_ptr()
         update.output, update.matched_key_end = output.data_ptr(), ends.data_ptr()
-        update.longest_total = max(old + new for old, new in zip(self._lengths, chunk_lengths))
-        workspace = cabi.router_update(update, self._device)
+        update.longest_total = longest_total
+        update.workspace, update.workspace_bytes = None, 0
+        workspace = cabi.router_update(update, self._device, stream)
         # stream-ordered launches: keep what they read alive until they have run
         for held in (tables, workspace):
             if held is not None:
-                held.record_stream(torch.cuda.current_stream(self._device))
+                held.record_stream(stream)
         self._device_lengths, self._device_lengths_next = \
             self._device_lengths_next, self._device_lengths
-        self._lengths = [old + new for old, new in zip(self._lengths, chunk_lengths)]
+        self._lengths = lengths
         return output, ends
 
 
