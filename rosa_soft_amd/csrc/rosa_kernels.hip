@@ -2677,12 +2677,19 @@ __global__ __launch_bounds__(kDecodeThreads) void router_decode_step_kernel(Rout
 // weights are the products' row operand, so that a lane ends up with four neighbouring
 // output columns of one token).  `weight` is the
 // [N][K] matrix of a linear layer (k contiguous), bfloat16; accumulation is float32.
-// A block of four waves computes 256 rows x 64 columns, each wave 64 x 64 (sixteen
-// 16 x 16 x 32 products per 32-wide k step).  Per staged step of 64 k (two products deep) a
+// A block of four waves computes 256 rows x 64 or 128 columns, each wave 64 rows (sixteen or
+// thirty-two 16 x 16 x 32 products per 32-wide k step).  Per staged step of 64 k (two products deep) a
 // block stages the weight tile [64][64] and, per row, the sign and validity bits of the step
 // in LDS; the loads of the next step are in flight while the products of this one run.
 constexpr int kProjectRows = 256;
 constexpr int kProjectColumns = 64;
+// Blocks of twice the columns expand every sign byte for eight products instead of four, which
+// halves the expansion (table reads, vector instructions) and the LDS traffic per product.
+// They are used where they fill the chip (two per compute unit): 8192 tokens x 2048 x 2048
+// (512 such blocks) 82 us with narrow blocks, 75 with wide ones; 4096 tokens (256) 46 and 54.
+// Value widths 16 and those not loaded by groups keep the narrow ones (the wide form is out of
+// registers there).
+constexpr int64_t kProjectWideBlocksMin = 512;
 constexpr int kProjectStep = 32;    // k of one matrix product, and what K must be a multiple of
 // k staged per barrier (128 needs registers beyond three waves per SIMD, and is slower for it)
 constexpr int kProjectStage = 64;
@@ -2743,9 +2750,36 @@ __device__ __forceinline__ uint2 ternary_step_bits(const ProjectParams& P, int64
   return make_uint2(signs, valid);
 }
 
-template <int HEADS>
-__global__ __launch_bounds__(256) void project_routed_bits_kernel(ProjectParams P) {
-  __shared__ __attribute__((aligned(16))) uint16_t weight_tile[2][kProjectColumns * kProjectWeightPitch];
+// The words of four steps of one token (a group) and the flags of the heads they belong to, for
+// widths that are a multiple of 32: one 16-byte load and one of up to four flags, where a load per
+// step and flag touches as many cache lines each (a line per token, at one per cycle, they took as
+// long as the products: 16384 tokens x 2048 x 2048 213 us, by groups 150, with blocks of 128
+// columns 146, of which the products need 55 at the dense bf16 peak).  Needs whole groups per token (H * nvw a multiple of 4) and heads that do
+// not end inside a group's halves (nvw 1, 2 or a multiple of 4).
+struct TernaryGroup {
+  uint4 words;
+  uint32_t flags;
+};
+
+__device__ __forceinline__ TernaryGroup load_ternary_group(const ProjectParams& P, int64_t token,
+                                                           int group) {
+  TernaryGroup loaded = {make_uint4(0u, 0u, 0u, 0u), 0u};
+  if (token < P.tokens) {
+    loaded.words = *reinterpret_cast<const uint4*>(P.sign_words + token * P.H * P.nvw + 4 * group);
+    const uint8_t* flags = P.routed + token * P.H + 4 * group / P.nvw;
+    if (P.nvw == 1) loaded.flags = *reinterpret_cast<const uint32_t*>(flags);
+    else if (P.nvw == 2) loaded.flags = *reinterpret_cast<const uint16_t*>(flags);
+    else loaded.flags = *flags;
+  }
+  return loaded;
+}
+
+// HEADS 1: as 0, by groups.
+// TILES: 16-column tiles of a block (and of each of its waves): 4 or 8.
+template <int HEADS, int TILES>
+__global__ __launch_bounds__(256, TILES > 4 ? 2 : 1) void project_routed_bits_kernel(ProjectParams P) {
+  constexpr int kColumns = 16 * TILES;
+  __shared__ __attribute__((aligned(16))) uint16_t weight_tile[2][kColumns * kProjectWeightPitch];
   // (signs, valid) of every product of the stage, per row
   __shared__ __attribute__((aligned(16))) uint2 row_bits[2][kProjectRows][kStageProducts];
   __shared__ __attribute__((aligned(8))) uint32_t ternary_table[kTernaryTableWords];
@@ -2757,38 +2791,67 @@ __global__ __launch_bounds__(256) void project_routed_bits_kernel(ProjectParams 
   // neighbouring blocks share their weight columns (same blockIdx.y) and follow each other
   // in row order, so the weight tiles of a column block stay in the cache of their XCD
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kProjectRows;
-  const int n0 = blockIdx.y * kProjectColumns;
+  const int n0 = blockIdx.y * kColumns;
   fill_ternary_table(ternary_table, thread);
 
-  v4f acc[4][4];
+  v4f acc[4][TILES];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < TILES; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   }
   const int products = P.K / kProjectStep;           // 32-wide k steps in all
   const int stages = (products + kStageProducts - 1) / kStageProducts;
-  // what a thread stages per stage: a quarter of one weight row's stage and one row's bits
+  // what a thread stages per stage: a quarter of every 64th weight row's stage and one row's bits
+  constexpr int kWeightRows = kColumns / 64;
   constexpr int kThreadElements = kProjectStage / 4;
   constexpr int kThreadChunks = kThreadElements / 8;   // of 16 bytes
   const int stage_n = thread >> 2;
   const int stage_k = (thread & 3) * kThreadElements;
   const uint16_t* weight_row = P.weight + static_cast<int64_t>(n0 + stage_n) * P.K + stage_k;
-  uint4 weight_in[kThreadChunks];
+  uint4 weight_in[kWeightRows][kThreadChunks];
   uint2 bits_in[kStageProducts];
+  static_assert(kStageProducts == 2, "a group holds two stages");
+  TernaryGroup group_in, group_now;  // HEADS 1
+  const int flag_shift = P.nvw == 1 ? 0 : P.nvw == 2 ? 1 : 2;
   const auto fetch_stage = [&](int stage) {
     // (K is a multiple of 32: the last stage may hold fewer products than the others)
 #pragma unroll
     for (int chunk = 0; chunk < kThreadChunks; ++chunk) {
       const int k = stage * kProjectStage + stage_k + 8 * chunk;
-      weight_in[chunk] = k + 8 <= P.K
-                             ? *reinterpret_cast<const uint4*>(weight_row + stage * kProjectStage + 8 * chunk)
-                             : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int r = 0; r < kWeightRows; ++r) {
+        weight_in[r][chunk] =
+            k + 8 <= P.K ? *reinterpret_cast<const uint4*>(weight_row + static_cast<int64_t>(64 * r) * P.K +
+                                                           stage * kProjectStage + 8 * chunk)
+                         : make_uint4(0u, 0u, 0u, 0u);
+      }
+    }
+    if constexpr (HEADS == 1) {
+      if ((stage & 1) == 0) group_in = load_ternary_group(P, row0 + thread, stage >> 1);
+      return;
+    }
+    if constexpr (HEADS == 2) {
+      if (P.H % 4 == 0) {  // the four heads of the stage in one load each, as in a group
+        uint4 words = make_uint4(0u, 0u, 0u, 0u);
+        uint32_t flags = 0u;
+        if (row0 + thread < P.tokens) {
+          const int64_t first = (row0 + thread) * P.H + 4 * stage;
+          words = *reinterpret_cast<const uint4*>(P.sign_words + first);
+          flags = *reinterpret_cast<const uint32_t*>(P.routed + first);
+        }
+        const auto head_mask = [&](int head) {
+          return ((flags >> (8 * head)) & 0xffu) == 1u ? 0xffffu : 0u;
+        };
+        bits_in[0] = make_uint2((words.x & 0xffffu) | (words.y << 16), head_mask(0) | (head_mask(1) << 16));
+        bits_in[1] = make_uint2((words.z & 0xffffu) | (words.w << 16), head_mask(2) | (head_mask(3) << 16));
+        return;
+      }
     }
 #pragma unroll
     for (int h = 0; h < kStageProducts; ++h) {
       const int step = stage * kStageProducts + h;
-      bits_in[h] = step < products ? ternary_step_bits<HEADS>(P, row0 + thread, step) : make_uint2(0u, 0u);
+      bits_in[h] = step < products ? ternary_step_bits<HEADS == 1 ? 0 : HEADS>(P, row0 + thread, step) : make_uint2(0u, 0u);
     }
   };
   fetch_stage(0);
@@ -2796,17 +2859,32 @@ __global__ __launch_bounds__(256) void project_routed_bits_kernel(ProjectParams 
     const int buffer = stage & 1;
     uint16_t* staged = &weight_tile[buffer][stage_n * kProjectWeightPitch + stage_k];
 #pragma unroll
-    for (int chunk = 0; chunk < kThreadChunks; ++chunk)
-      *reinterpret_cast<uint4*>(staged + 8 * chunk) = weight_in[chunk];
+    for (int r = 0; r < kWeightRows; ++r) {
+#pragma unroll
+      for (int chunk = 0; chunk < kThreadChunks; ++chunk)
+        *reinterpret_cast<uint4*>(staged + 64 * r * kProjectWeightPitch + 8 * chunk) =
+            weight_in[r][chunk];
+    }
+    if constexpr (HEADS == 1) {
+      if ((stage & 1) == 0) group_now = group_in;
+      const int step = 2 * (stage & 1);  // of the group
+      const uint32_t words[2] = {step == 0 ? group_now.words.x : group_now.words.z,
+                                 step == 0 ? group_now.words.y : group_now.words.w};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t flag = (group_now.flags >> (8 * ((step + h) >> flag_shift))) & 0xffu;
+        bits_in[h] = make_uint2(words[h], flag == 1u ? 0xffffffffu : 0u);
+      }
+    }
 #pragma unroll
     for (int h = 0; h < kStageProducts; ++h) row_bits[buffer][thread][h] = bits_in[h];
     __syncthreads();
     if (stage + 1 < stages) fetch_stage(stage + 1);  // in flight during the products
 #pragma unroll
     for (int h = 0; h < kStageProducts; ++h) {
-      v4u b_operand[4];
+      v4u b_operand[TILES];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < TILES; ++j) {
         b_operand[j] = *reinterpret_cast<const v4u*>(
             &weight_tile[buffer][(16 * j + li) * kProjectWeightPitch + kProjectStep * h + 8 * lg]);
       }
@@ -2823,7 +2901,7 @@ __global__ __launch_bounds__(256) void project_routed_bits_kernel(ProjectParams 
         // (the weights as the row operand: a lane then holds four neighbouring output
         // columns of one token, which leave as one 8-byte store)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16(b_operand[j], a_operand, acc[i][j]);
+        for (int j = 0; j < TILES; ++j) acc[i][j] = mfma_bf16(b_operand[j], a_operand, acc[i][j]);
       }
     }
   }
@@ -2834,7 +2912,7 @@ __global__ __launch_bounds__(256) void project_routed_bits_kernel(ProjectParams 
     const int64_t token = row0 + wave * 64 + 16 * i + li;
     if (token >= P.tokens) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TILES; ++j) {
       const int64_t index = token * P.N + n0 + 16 * j + 4 * lg;
       v4f value = acc[i][j];
       if (P.residual != nullptr) {
@@ -3066,15 +3144,18 @@ int rosa_hip_project_routed_bits(const uint32_t* sign_words, const uint8_t* rout
       misaligned(out, 8) || misaligned(residual, 8))
     return fail(1, "project_routed_bits: weight and sign_words must be 16-byte aligned, out and "
                    "residual 8-byte, routed 4-byte");
-  const dim3 grid(static_cast<unsigned>(row_blocks), static_cast<unsigned>(N / kProjectColumns));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (Dv == 8) {
-    hipLaunchKernelGGL(project_routed_bits_kernel<4>, grid, dim3(256), 0, s, P);
-  } else if (Dv == 16) {
-    hipLaunchKernelGGL(project_routed_bits_kernel<2>, grid, dim3(256), 0, s, P);
-  } else {
-    hipLaunchKernelGGL(project_routed_bits_kernel<0>, grid, dim3(256), 0, s, P);
-  }
+  const bool grouped = Dv >= 32 && (H * P.nvw) % 4 == 0 && (P.nvw <= 2 || P.nvw % 4 == 0);
+  const bool wide = (Dv == 8 || grouped) && N % (2 * kProjectColumns) == 0 &&
+                    row_blocks * (N / (2 * kProjectColumns)) >= kProjectWideBlocksMin;
+  const dim3 grid(static_cast<unsigned>(row_blocks),
+                  static_cast<unsigned>(N / (wide ? 2 * kProjectColumns : kProjectColumns)));
+  const auto kernel =
+      Dv == 8    ? (wide ? project_routed_bits_kernel<4, 8> : project_routed_bits_kernel<4, 4>)
+      : Dv == 16 ? project_routed_bits_kernel<2, 4>
+      : grouped  ? (wide ? project_routed_bits_kernel<1, 8> : project_routed_bits_kernel<1, 4>)
+                 : project_routed_bits_kernel<0, 4>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, P);
   const hipError_t launch = hipGetLastError();
   if (launch != hipSuccess) return fail_hip(launch, "project_routed_bits launch");
   return 0;

@@ -86,6 +86,37 @@ def test_projection_of_the_bit_form_matches_the_expanded_product(cabi, heads, va
     torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=1e-6 * float(want.abs().max()))
 
 
+@pytest.mark.parametrize("heads,value_dim,width,tokens", [
+    (4, 32, 64, 257),       # whole groups of four steps, a head per step
+    (2, 64, 128, 255),      # ... two steps per head
+    (1, 128, 64, 33),       # ... one head per group
+    (3, 128, 64, 300),      # ... odd heads, whole groups all the same
+    (6, 32, 64, 256),       # half a group left over: step by step
+    (4, 96, 64, 100),       # heads that end inside a group: step by step
+    (4, 16, 64, 1),         # the four heads of a stage at once
+    (6, 16, 192, 290),      # half a stage left over
+    (4, 32, 2048, 8001),    # 512 blocks of 128 columns, the last one with a row block cut short
+    (4, 32, 2048, 7936),    # one row block fewer: blocks of 64 columns
+    (8, 8, 2048, 8192),     # 128 columns, four heads per step
+])
+def test_projection_by_groups_and_by_wide_blocks(cabi, heads, value_dim, width, tokens):
+    device = torch.device("cuda:0")
+    generator = torch.Generator(device=device).manual_seed(5)
+    words = (value_dim + 31) // 32
+    sign_words = torch.randint(-2**31, 2**31, (1, tokens, heads, words), device=device,
+                               generator=generator).to(torch.int32)
+    if value_dim < 32:
+        sign_words &= (1 << value_dim) - 1
+    routed = (torch.rand(1, tokens, heads, device=device, generator=generator) < 0.7).to(torch.uint8)
+    weight = (torch.randn(width, heads * value_dim, device=device, generator=generator) /
+              (heads * value_dim) ** 0.5).to(torch.bfloat16)
+    residual = torch.randn(1, tokens, width, device=device, generator=generator).to(torch.bfloat16)
+    got = cabi.project_routed_bits(sign_words, routed, value_dim, weight, residual)
+    want = _projection_reference(cabi, sign_words, routed, value_dim, weight, residual)
+    # as above: exact products, float32 sums, one rounding to bfloat16
+    torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=1e-6 * float(want.abs().max()))
+
+
 def test_projection_at_the_shape_of_configuration_3(cabi):
     device = torch.device("cuda:0")
     query, key, value = _inputs((4, 4096, 32, 16), (4, 4096, 32, 64), torch.bfloat16, 33)
