@@ -2420,15 +2420,20 @@ __global__ __launch_bounds__(kWave) void router_candidates_kernel(RouterUpdate U
   const int walk_budget = budget / 4;
   int spent = 0, walked = 0;  // wave-uniform
   uint64_t best = 0;          // (run << 32) | route
-  // A lane walks its bucket through dependent round trips to the index, so it keeps the next
-  // four entries in flight (one at a time: 32 us where this takes 18, 2 slots x 64 heads x
-  // 4096 tokens; 8 slots 122 us before the routes went out run-major, now 57).
+  // A lane walks its bucket through dependent loads of a cache line per lane, 64 cycles of the
+  // address unit each: four entries of one word come in one (one entry per load, 2 slots x 64
+  // heads x 4096 tokens: 32 us one at a time, 18 four in flight, 13 so).  The last
+  // load of a run may reach past its entries, into what follows them in the workspace.
   constexpr int kAhead = 4;
-  typename Entry::Word ahead[kAhead];
+  typename Entry::Word ahead[kAhead] = {};
   const auto fetch = [&](int first) {
+    if constexpr (NARROW) {
+      if (first < end) __builtin_memcpy(ahead, routes + first, sizeof(ahead));
+    } else {
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      ahead[j] = first + j < end ? routes[first + j] : Entry::make(0u, 0x100u);
+      for (int j = 0; j < kAhead; ++j) {
+        ahead[j] = first + j < end ? routes[first + j] : Entry::make(0u, 0x100u);
+      }
     }
   };
   bool beyond = false;  // the entries left belong to passes that begin beyond this row
