@@ -216,3 +216,27 @@ def test_indexed_forward_of_one_long_sequence_equals_the_scan(cabi, bits):
         cabi.set_forward_index(None)
     assert int((want_routes > 0).sum()) > length // 4
     assert torch.equal(routes, want_routes) and torch.equal(output, want_output)
+
+
+@pytest.mark.parametrize("bits,length", [(6, 515), (8, 1027), (8, 2049), (12, 16400)])
+def test_words_with_bits_beyond_the_width_route_as_the_scan_does(cabi, bits, length):
+    # words the caller packed are compared whole, so they keep entries of four words; the
+    # operator's own words (one-word entries here) give the scan's routes as well
+    query, key = (part.to("cuda:0") for part in _pattern_inputs("random", 1, length, 2, bits, 77))
+    value = nonzero_randn((1, length, 2, 8), dtype=torch.float32, seed=80).to("cuda:0")
+    output, packed_query, packed_key, routes = cabi.hard_forward(query, key, value, 19)
+    stray_query = packed_query | (torch.arange(length, device="cuda:0") % 3 << 13).to(torch.int32)
+    stray_key = packed_key | (torch.arange(length, device="cuda:0") % 2 << 13).to(torch.int32)
+    results = []
+    for mode in (None, "scan"):
+        cabi.set_forward_index(mode)
+        try:
+            own = cabi.hard_forward(query, key, value, 19)
+            stray = cabi.hard_forward_words(stray_query, stray_key, value, 19, symbol_bits=bits)
+        finally:
+            cabi.set_forward_index(None)
+        results.append((own[0], own[3], *stray))
+    for indexed, scanned in zip(*results):
+        assert torch.equal(indexed, scanned)
+    assert torch.equal(results[0][0], output) and torch.equal(results[0][1], routes)
+    assert not torch.equal(results[0][3], routes)
