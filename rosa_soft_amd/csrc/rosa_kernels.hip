@@ -1035,6 +1035,62 @@ __device__ __forceinline__ void prepare_grad_rows(
   for (int k = terms * dvp + d; k < pitch; k += dvp) row[k] = uint16_t(0);
 }
 
+// Eight neighbouring elements in 16-byte loads (`first` and the tensor suitably aligned).
+template <int DTYPE>
+__device__ __forceinline__ void load_eight(const void* __restrict__ data, int64_t first,
+                                           float (&values)[8]) {
+  if constexpr (DTYPE == ROSA_DTYPE_F32) {
+    const float4* source = reinterpret_cast<const float4*>(static_cast<const float*>(data) + first);
+    const float4 low = source[0], high = source[1];
+    values[0] = low.x; values[1] = low.y; values[2] = low.z; values[3] = low.w;
+    values[4] = high.x; values[5] = high.y; values[6] = high.z; values[7] = high.w;
+  } else {
+    const uint4 raw = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(data) + first);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) values[j] = load_as_float<DTYPE>(&raw, j);
+  }
+}
+
+// prepare_grad_rows for whole pieces of eight elements: one thread per piece, 16-byte loads and
+// stores, the row's numbering (several divisions) once per eight elements.
+template <int DTYPE>
+__device__ __forceinline__ void prepare_grad_pieces(
+    int64_t index, const void* __restrict__ grad_output, uint16_t* __restrict__ grad_rows,
+    int64_t rows, int H, int Dv, int dvp, int T, int N, int varlen, int value_stride,
+    int value_offset, int terms, int pitch) {
+  const int row_pieces = dvp / 8;  // a power of two
+  const int log_pieces = 31 - __clz(row_pieces);
+  if (index >= rows * row_pieces) return;
+  const int64_t dst = index >> log_pieces;  // head-major row
+  const int d = 8 * static_cast<int>(index & (row_pieces - 1));
+  int64_t source_row;  // token * H + h
+  if (varlen) {
+    const int64_t h = dst / N;
+    source_row = (dst - h * N) * H + h;
+  } else {
+    const int64_t bh = dst / T;
+    const int64_t b = bh / H;
+    source_row = (b * T + (dst - bh * T)) * H + (bh - b * H);
+  }
+  float rest[8] = {};
+  if (d < Dv) load_eight<DTYPE>(grad_output, source_row * value_stride + value_offset + d, rest);
+  uint16_t* row = grad_rows + dst * pitch;
+  for (int t = 0; t < terms; ++t) {
+    uint32_t term[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      term[j] = bf16_nearest(rest[j]);
+      // (as above: exact; an infinite or NaN term ends the series)
+      rest[j] = (term[j] & 0x7f80u) == 0x7f80u ? 0.0f : rest[j] - __uint_as_float(term[j] << 16);
+    }
+    *reinterpret_cast<uint4*>(row + t * dvp + d) =
+        make_uint4((term[0] & 0xffffu) | (term[1] << 16), (term[2] & 0xffffu) | (term[3] << 16),
+                   (term[4] & 0xffffu) | (term[5] << 16), (term[6] & 0xffffu) | (term[7] << 16));
+  }
+  for (int k = terms * dvp + d; k < pitch; k += dvp)
+    *reinterpret_cast<uint4*>(row + k) = make_uint4(0u, 0u, 0u, 0u);
+}
+
 __device__ __forceinline__ int64_t value_word_row(int64_t row, int Hv, int T, int N, int varlen) {
   const int64_t token = row / Hv;  // row = token * Hv + hv
   const int64_t hv = row - token * Hv;
@@ -1083,6 +1139,28 @@ __device__ __forceinline__ void pack_value_bits_rows(
     }
     value_bits[dst * nvw + w] = word;
   }
+}
+
+// ... for whole pieces of eight elements: one thread per word.
+template <int DTYPE>
+__device__ __forceinline__ void pack_value_bits_words(
+    int64_t index, const void* __restrict__ value, uint32_t* __restrict__ value_bits, int64_t rows,
+    int Hv, int Dv, int nvw, int T, int N, int varlen, int value_stride, int value_offset) {
+  if (index >= rows * nvw) return;
+  const int64_t row = nvw == 1 ? index : index / nvw;
+  const int w = static_cast<int>(index - row * nvw);
+  uint32_t word = 0u;
+#pragma unroll
+  for (int piece = 0; piece < 4; ++piece) {
+    const int d = 32 * w + 8 * piece;
+    if (d < Dv) {
+      float values[8];
+      load_eight<DTYPE>(value, row * value_stride + value_offset + d, values);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) word |= values[j] > 0.0f ? 1u << (8 * piece + j) : 0u;
+    }
+  }
+  value_bits[value_word_row(row, Hv, T, N, varlen) * nvw + w] = word;
 }
 
 // Per row: the reference point of the softmax exponent and the constant part
@@ -1141,6 +1219,10 @@ struct PrepareParams {
   float scale;
   int analytic;
   int ballot;  // value width is 8, 16, 32 or 64: pack signs with wave ballots
+  // Widths of whole, 16-byte aligned pieces of eight elements (of grad_output; of the values):
+  // a thread per piece or word.  Per element, 16384 rows x 32 heads x 64 bfloat16 took 237 us of
+  // numbering and two-byte accesses where the bytes need about 60; by pieces 76.
+  int grad_pieces, value_pieces;
   float* fill[3];  // gradient buffers to clear (null: none), with their lengths
   int64_t fill_elements[3];
   unsigned grad_blocks, value_blocks, stats_blocks, fill_blocks;
@@ -1151,6 +1233,12 @@ __global__ __launch_bounds__(256) void vjp_prepare_kernel(PrepareParams p) {
   unsigned block = blockIdx.x;
   const auto element = [&]() { return static_cast<int64_t>(block) * blockDim.x + threadIdx.x; };
   if (block < p.grad_blocks) {
+    if (p.grad_pieces) {
+      prepare_grad_pieces<DTYPE>(element(), p.grad_output, p.grad_rows, p.symbol_rows, p.L.H, p.Dv,
+                                 p.dvp, p.L.T, p.L.N, p.L.varlen, p.value_stride, p.value_offset,
+                                 p.grad_terms, p.grad_pitch);
+      return;
+    }
     prepare_grad_rows<DTYPE>(element(), p.grad_output, p.grad_rows, p.symbol_rows, p.L.H, p.Dv,
                              p.dvp, p.L.T, p.L.N, p.L.varlen, p.value_stride, p.value_offset,
                              p.grad_terms, p.grad_pitch);
@@ -1158,7 +1246,11 @@ __global__ __launch_bounds__(256) void vjp_prepare_kernel(PrepareParams p) {
   }
   block -= p.grad_blocks;
   if (block < p.value_blocks) {
-    if (p.ballot) {
+    if (p.value_pieces) {
+      pack_value_bits_words<DTYPE>(element(), p.value, p.value_bits, p.value_rows, p.L.Hv, p.Dv,
+                                   p.nvw, p.L.T, p.L.N, p.L.varlen, p.value_stride,
+                                   p.value_offset);
+    } else if (p.ballot) {
       pack_value_bits_ballot<DTYPE>(element(), p.value, p.value_bits, p.value_rows, p.L.Hv, p.Dv,
                                     p.nvw, p.L.T, p.L.N, p.L.varlen, p.value_stride,
                                     p.value_offset);
@@ -1178,7 +1270,13 @@ __global__ __launch_bounds__(256) void vjp_prepare_kernel(PrepareParams p) {
   const int64_t stride = static_cast<int64_t>(p.fill_blocks) * blockDim.x;
   for (int part = 0; part < 3; ++part) {
     if (p.fill[part] == nullptr) continue;
-    for (int64_t i = element(); i < p.fill_elements[part]; i += stride) p.fill[part][i] = 0.0f;
+    const int64_t wide = (reinterpret_cast<uintptr_t>(p.fill[part]) & 15) == 0
+                             ? p.fill_elements[part] / 4 : 0;  // in 16-byte stores
+    float4* quads = reinterpret_cast<float4*>(p.fill[part]);
+    for (int64_t i = element(); i < wide; i += stride)
+      quads[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int64_t i = 4 * wide + element(); i < p.fill_elements[part]; i += stride)
+      p.fill[part][i] = 0.0f;
   }
 }
 
@@ -1992,9 +2090,18 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
       prepare.scale = scale;
       prepare.analytic = analytic ? 1 : 0;
       prepare.ballot = (L.Dv == 8 || L.Dv == 16 || L.Dv == 32 || L.Dv == 64) ? 1 : 0;
-      prepare.grad_blocks = blocks_for(view.symbol_rows * dvp, 256);
-      prepare.value_blocks =
-          blocks_for(prepare.ballot ? view.value_rows * L.Dv : view.value_rows, 256);
+      const auto whole_pieces = [&](const void* data) {
+        const int64_t item = DTYPE == ROSA_DTYPE_F32 ? 4 : 2;
+        return L.Dv % 8 == 0 && full_width % 8 == 0 && value_offset % 8 == 0 &&
+               (reinterpret_cast<uintptr_t>(data) & 15) == 0 && full_width * item % 16 == 0;
+      };
+      prepare.grad_pieces = whole_pieces(grad_output) ? 1 : 0;
+      prepare.value_pieces = whole_pieces(value) ? 1 : 0;
+      prepare.grad_blocks =
+          blocks_for(view.symbol_rows * (prepare.grad_pieces ? dvp / 8 : dvp), 256);
+      prepare.value_blocks = blocks_for(prepare.value_pieces ? view.value_rows * prepare.nvw
+                                        : prepare.ballot     ? view.value_rows * L.Dv
+                                                             : view.value_rows, 256);
       prepare.stats_blocks = blocks_for(view.symbol_rows, 256);
       if (value_offset == 0) {  // the gradient buffers are cleared once, before the first slice
         // what the gradient kernel adds into: the tensors, or the head-major accumulators

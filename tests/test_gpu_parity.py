@@ -730,3 +730,37 @@ def test_value_gradient_keeps_its_margin_with_split_weights(cabi, c_oracle, T, H
     assert_gradients_close(grads[2], want[2], "dv", slack=0.7)
     assert_gradients_close(grads[0], want[0], "dq")
     assert_gradients_close(grads[1], want[1], "dk")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("width", [8, 24, 40, 64, 72])
+def test_backward_inputs_off_their_alignment_give_the_same_gradients(dtype, width):
+    # widths of whole eight-element pieces are prepared in 16-byte accesses where the tensors
+    # allow it; one element off that alignment they are prepared element by element.  Values are
+    # the same, so the gradients differ by the order of the float32 atomics only.
+    import rosa_soft_amd
+
+    device = torch.device("cuda:0")
+    generator = torch.Generator(device=device).manual_seed(11)
+    randn = lambda *shape: torch.randn(*shape, device=device, generator=generator).to(dtype)
+    query, key = randn(2, 150, 4, 6), randn(2, 150, 4, 6)
+    value, grad_output = randn(2, 150, 2, width), randn(2, 150, 4, width)
+
+    def shifted(tensor):
+        storage = torch.empty(tensor.numel() + 1, dtype=tensor.dtype, device=device)
+        view = storage[1:].view(tensor.shape)
+        view.copy_(tensor)
+        assert view.is_contiguous() and view.data_ptr() % 16 != 0
+        return view
+
+    results = []
+    for place in (lambda tensor: tensor.clone(), shifted):
+        leaves = [query.clone().requires_grad_(), key.clone().requires_grad_(),
+                  place(value).requires_grad_()]
+        output = rosa_soft_amd.rosa_soft(*leaves, max_suffix_length=20)
+        results.append(torch.autograd.grad(output, leaves, place(grad_output)))
+    for aligned, off in zip(*results):
+        difference = (aligned.float() - off.float()).norm() / aligned.float().norm()
+        # float32 sums in another order: 1e-6; the narrow types round near ties the other way
+        bound = 1e-5 if dtype == torch.float32 else 1e-3
+        assert float(difference) < bound, float(difference)
