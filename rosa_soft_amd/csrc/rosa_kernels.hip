@@ -2208,6 +2208,7 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
           std::log2(static_cast<float>(longest));
       P.tail_threshold = std::exp2(std::max(exponent, -120.0f));
     }
+    P.halo_decay = (128.0f + 150.0f + std::log2(2.0f * (static_cast<float>(L.W) + 1.0f))) / P.gate_log2;
     P.gradient_mask = gradient_mask;
     P.dvp = dvp;
     P.grad_query = sum_query;

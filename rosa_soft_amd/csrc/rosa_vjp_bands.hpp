@@ -60,6 +60,11 @@ struct VjpParams {
   const int32_t* gradient_prefix;  // packed: pieces before each sequence
   const int32_t* stats_prefix;
   int gradient_pieces;          // the gradient pass runs in pieces: it reads chunk_decay
+  // mismatching bits on a diagonal below a piece beyond which nothing can reach the piece: the
+  // carry is below 2^128, it enters an adjoint times at most W + 1 and so does the sum of the
+  // overflow terms, and below 2^-150 nothing is left of a float32.  (A bound relative to the
+  // carry, 2^-34 of it and the like, is not enough: rows of grad_output may differ by any factor.)
+  float halo_decay;
   int single_form;              // only the three-term form of the gradient kernel is launched
   uint16_t* chunk_decay;        // per chunk record: fewest mismatching bits any diagonal of the band
                                 // meets in the chunk's 16 rows
@@ -1432,11 +1437,12 @@ void vjp_gradients_kernel(VjpParams P) {
       int halo = 0;
       if (want_qk) {
         // At most the W - 1 rows of the horizon, and no more chunks than it takes for the gates
-        // of every diagonal to multiply to nothing: the carry that crosses them, and every
-        // overflow term whose window holds them, is then below `tail_threshold` of its value.
-        // Random symbols need one or two chunks, whatever the window.
+        // of every diagonal to multiply to so little that whatever finite carry comes from the
+        // rows below, what is left of it (and of every overflow term whose window holds these
+        // rows) is below the smallest float32: see halo_decay.  Random symbols of eight bits
+        // need eleven chunks at mismatch_scale 3 and four at 9, whatever the window.
         const int most = (P.L.W - 1 + kChunk - 1) / kChunk;
-        const float enough = -__log2f(P.tail_threshold) / P.gate_log2;
+        const float enough = P.halo_decay;
         float met = 0.0f;
         int chunks = 0;
         while (chunks < most && met < enough && row_end + kChunk * chunks < view.steps) {

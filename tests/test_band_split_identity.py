@@ -78,3 +78,33 @@ def test_a_walk_started_below_a_cut_reproduces_the_rows_above_it(pattern, window
         if pattern == "all_match" and cut + window - 1 < n and window > 2:
             short = reverse_walk(gates, adjoint, evidence, overflow, window, cut + window - 2, 0)
             assert not np.allclose(short[:cut], whole[:cut], rtol=1e-10, atol=1e-12)
+
+
+@pytest.mark.parametrize("window", [24, 40])
+def test_a_halo_may_end_where_nothing_is_left_of_any_float32_carry(window):
+    """The halo may be cut short only where the gates below the cut multiply to less than
+    2^-278 / (2 W + 2): carries are below 2^128, and what then reaches the rows above is below
+    2^-150, half the smallest float32.  A bound relative to the carry (2^-34 / W^2 here) is not
+    one on the result: rows of the gradient of the output may differ by any factor."""
+
+    rng = np.random.default_rng(window)
+    n, cut = 60, 16
+    gates = np.exp2(-rng.integers(10, 21, n).astype(float))
+    adjoint = rng.standard_normal(n)
+
+    def halo_to(limit):
+        rows, product = 0, 1.0
+        while product >= limit:
+            product *= gates[cut + rows]
+            rows += 1
+        return cut + rows
+
+    exact, relative = halo_to(2.0 ** -278 / (2 * window + 2)), halo_to(2.0 ** -34 / window ** 2)
+    assert relative < exact < cut + window - 1
+    adjoint[relative:] *= 1e30
+    evidence, overflow = forward(gates, window)
+    whole = reverse_walk(gates, adjoint, evidence, overflow, window, n, 0)
+    piece = reverse_walk(gates, adjoint, evidence, overflow, window, exact, 0)
+    np.testing.assert_allclose(piece[:cut], whole[:cut], rtol=1e-12, atol=2.0 ** -149)
+    short = reverse_walk(gates, adjoint, evidence, overflow, window, relative, 0)
+    assert not np.allclose(short[:cut], whole[:cut], rtol=1e-6, atol=0.0)

@@ -664,6 +664,62 @@ def test_bands_cut_into_pieces_match_oracle(cabi, c_oracle, records, B, T, H, D,
         assert_gradients_close(got, unsplit.cpu(), name + " against whole bands", slack)
 
 
+def query_gradient_of_any_range(query, key, value, grad_output, W, ms):
+    """dQ of one sequence and head in float64, every adjoint's share of a row as a sum of positive
+    products (the streamed oracle takes the tail of a score by subtraction, which loses shares
+    2^-53 and less of it)."""
+
+    query, key, value, go = (x[0, :, 0].double() for x in (query, key, value, grad_output))
+    T, D = query.shape
+    q_sign, k_sign, v_sign = ((x > 0).double() * 2.0 - 1.0 for x in (query, key, value))
+    mismatches = (D - q_sign @ k_sign.t()) / 2                       # [t, key position]
+    gates = torch.exp(-ms * mismatches / D)
+    grad = torch.zeros(T, D, dtype=torch.float64)
+    for t in range(1, T):
+        routes = torch.arange(1, t + 1)
+        steps = torch.arange(min(W, t))
+        positions = routes[:, None] - 1 - steps                      # of the keys of every suffix
+        live = positions >= 0
+        factors = torch.where(live, gates[t - steps[None, :], positions.clamp_min(0)], 0.0)
+        products = torch.cumprod(factors, dim=1)
+        tails = products.flip(1).cumsum(1).flip(1)                   # sum of the products from j on
+        root = torch.sqrt(1.0 + tails[:, 0])
+        logits = 2.414213562373095 * (root - 1.0) - np.log(t)
+        weights = torch.exp(logits)
+        probability = weights / (weights.sum() + np.exp(0.5))
+        utility = v_sign[routes] @ go[t]
+        adjoint = probability * (utility - probability @ utility) * 0.5 * 2.414213562373095 / root
+        shares = 0.5 * ms / D * adjoint[:, None] * tails              # [route, step back]
+        for j in steps.tolist():
+            grad[t - j] += shares[:, j] @ k_sign[(routes - 1 - j).clamp_min(0)]
+    return grad / (1.0 + query.abs()) ** 2
+
+
+@pytest.mark.parametrize("D,W,ms,gap", [(8, 64, 3.0, 50), (8, 200, 3.0, 50), (4, 150, 9.0, 18),
+                                        (2, 120, 3.0, 50)])
+def test_a_piece_sees_carries_of_any_size_below_it(cabi, D, W, ms, gap):
+    """Rows of grad_output may differ by any factor.  Here those from `gap` rows below the first
+    cut on are 1e30 times the ones above it, so that what reaches the rows above the cut through
+    that many gates is still of their own adjoints' size or above: every row of dQ, measured
+    against its own largest element and not the tensor's, comes out as float64 has it.
+    (5e-4: a factor 2^-k of the gates carries the rounding of its exponent, k ln 2 times 2^-24,
+    once per gate, and k here is a few hundred.)"""
+
+    T, rows = 330, 64
+    query, key, value, grad_output = make_case(1, T, 1, D, 1, 8, torch.float32, seed=7 * W + D)
+    grad_output[:, rows + 1 + gap:] *= 1e30
+    cabi.set_gradient_piece_rows(rows)
+    try:
+        *_, grads = run_device(cabi, query, key, value, grad_output, W, ms=ms)
+    finally:
+        cabi.set_gradient_piece_rows(None)
+    want = query_gradient_of_any_range(query, key, value, grad_output, W, ms)
+    got = grads[0].cpu().double()[0, :, 0]
+    scale = want.abs().amax(dim=1).clamp_min(1e-30)
+    worst = (got - want).abs().amax(dim=1) / scale
+    assert worst.max().item() <= 5e-4, (int(worst.argmax()), worst.max().item())
+
+
 @pytest.mark.parametrize("lengths,W,p,pattern", [
     ([33], 8, 0.0, "random"), ([34], 40, 0.1, "all_match"), ([65], 7, 0.0, "shifted"),
     ([98], 16, 0.1, "random"), ([129], 200, 0.0, "periodic"), ([193], 31, 0.1, "shifted"),
