@@ -267,19 +267,26 @@ __host__ __device__ inline int64_t checkpoint_slots(int64_t steps, int64_t bands
   return steps / 16 + bands + 1;
 }
 
-// Rows of a piece of a band (a multiple of `align`), 0 for whole bands: `band_rows` rows of all
-// bands together over `capacity` resident waves is what every wave would walk if the work
-// could be cut anywhere, and bands longer than that are cut into equal pieces of about that
-// length.  Never below `least` rows: what a piece costs beyond its own rows (the sweep in front
-// of it, the halo below it) is of that size.
-__host__ __device__ inline int piece_rows_for(int64_t band_rows, int longest, int64_t capacity,
-                                              int least, int align) {
-  const int64_t share = (band_rows + capacity - 1) / capacity;
-  const int64_t ideal = share > least ? share : least;
-  if (longest - 1 <= ideal) return 0;
-  const int64_t pieces = (longest - 1 + ideal - 1) / ideal;
-  const int64_t rows = (longest - 1 + pieces - 1) / pieces;
-  return static_cast<int>((rows + align - 1) / align * align);
+// Rows of a piece of a band (a multiple of `align`, never below `least`), 0 for whole bands.
+// `band_rows` rows of all `bands` bands over `capacity` resident waves are what every wave would
+// walk if the work could be cut anywhere; bands longer than that are cut so that about one piece
+// falls to a wave.  A tenth more than the share makes up for the pieces that end a band and are
+// shorter; at the share itself there are up to a third more pieces than waves and a second round
+// of full ones (gradient pass of 4096 tokens x 8 heads, W 64: 512 rows 241 us, 576 rows 197; of
+// 1500 x 16, 64 values: 256 rows 251 us, 320 rows 189).  Where every band has a wave of its own
+// halves are short enough: the waves that end first are those of the shortest bands, and take the
+// longest second halves (2 x 1024 tokens x 64 heads: 512 rows 210 us, 608 rows 231).
+// What a piece walks beyond its own rows (a halo below it or a sweep in front of it, W rows at
+// most) is left out: waves in parallel repeat it, and even where the window is the sequence and
+// every symbol matches, the smallest pieces are the fastest (2048 tokens x 2 heads, W 2048:
+// 64 rows 404 us, 512 rows 430, whole bands 525).
+__host__ __device__ inline int piece_rows_for(int64_t band_rows, int64_t bands, int longest,
+                                              int64_t capacity, int least, int align) {
+  int64_t ideal = (11 * band_rows + 10 * capacity - 1) / (10 * capacity);
+  if (bands <= capacity && ideal > longest / 2) ideal = longest / 2;
+  if (ideal < least) ideal = least;
+  const int64_t rows = (ideal + align - 1) / align * align;
+  return rows < longest - 1 ? static_cast<int>(rows) : 0;
 }
 
 __host__ __device__ inline int pieces_of_band(int piece_rows, int longest) {

@@ -166,9 +166,10 @@ __global__ void prepare_sequences_kernel(const int32_t* __restrict__ cu_seqlens,
       all_steps = scan(sums[0]);
       step_prefix[S] = all_steps;
       const int forced = pieces.forced_gradient_rows;
+      const int64_t bands = static_cast<int64_t>(block_prefix[S]) * H;
       plan[0] = forced != 0 ? max(forced, 0)
-          : piece_rows_for(all_steps * H, longest, pieces.gradient_waves, kPieceRowsMin, kPieceAlign);
-      plan[1] = piece_rows_for(all_steps * H, longest, pieces.stats_waves, kPieceRowsMin, kChunk);
+          : piece_rows_for(all_steps * H, bands, longest, pieces.gradient_waves, kPieceRowsMin, kPieceAlign);
+      plan[1] = piece_rows_for(all_steps * H, bands, longest, pieces.stats_waves, kPieceRowsMin, kChunk);
     }
     __syncthreads();
     const int gradient_rows = plan[0], stats_rows = plan[1];
@@ -1314,10 +1315,6 @@ int device_simds() {
 
 // blocks of the gradient kernel that are resident at two waves per SIMD
 int max_resident_blocks() { return 2 * device_simds(); }
-int resident_gradient_waves(int value_tiles, int symbol_tiles) {
-  return device_simds() * (gradient_waves(value_tiles, symbol_tiles) < 2
-                     ? 2 : gradient_waves(value_tiles, symbol_tiles));
-}
 
 // Waves per block of the gradient kernel (rosa_hip_set_gradient_block_waves overrides).
 // Two waves halve the column atomics, which bound the wide tiles; the narrow tile is bound
@@ -1331,44 +1328,10 @@ std::atomic<int> g_gradient_block_waves{0};  // 0: by shape
 // overrides): 0 by shape, -1 never, otherwise that many rows.
 std::atomic<int> g_gradient_piece_rows{0};
 
-// How the bands of the gradient kernel are cut into pieces (vjp_gradients_kernel): only with
-// single-wave blocks, and only where whole bands would leave resident waves idle (a band is
-// as long as its diagonal, so the kernel would last as long as its longest one).  A piece is a
-// whole number of staged segments; piece_rows_for says how long.
-struct PiecePlan {
-  int piece_rows;   // 0: whole bands
-  int max_pieces;   // work items per band
-};
-
 // rows of all bands of the problem; of a packed batch the most there can be (one sequence)
 int64_t band_rows_at_most(const Layout& L) {
   return L.varlen ? static_cast<int64_t>(L.H) * band_steps_total(L.N)
                   : static_cast<int64_t>(L.B) * L.H * band_steps_total(L.T);
-}
-
-PiecePlan plan_band_pieces(const Layout& L, int64_t resident_waves) {
-  PiecePlan plan{0, 1};
-  const int longest = L.varlen ? L.N : L.T;
-  const int64_t units = static_cast<int64_t>(L.slots) * L.H;
-  int rows = 0;
-  const int forced_rows = g_gradient_piece_rows.load(std::memory_order_relaxed);
-  if (forced_rows > 0) {
-    rows = (std::max(forced_rows, 2 * kPieceAlign) + kPieceAlign - 1) / kPieceAlign * kPieceAlign;
-    if (longest - 1 <= rows) rows = 0;
-  } else if (forced_rows == 0 && g_gradient_block_waves.load(std::memory_order_relaxed) != 2 &&
-             units < 2 * resident_waves) {
-    // (a packed batch is cut on the device, by its actual lengths; here it counts as equal
-    // sequences)
-    const int64_t rows_in_all =
-        L.varlen ? static_cast<int64_t>(L.H) * L.S * band_steps_total(L.N / std::max(L.S, 1))
-                 : band_rows_at_most(L);
-    rows = piece_rows_for(rows_in_all, longest, resident_waves, kPieceRowsMin, kPieceAlign);
-  }
-  const int pieces = pieces_of_band(rows, longest);
-  if (rows <= 0 || pieces < 2 || units * pieces > INT32_MAX) return plan;
-  plan.piece_rows = rows;
-  plan.max_pieces = pieces;
-  return plan;
 }
 
 // waves of the row-statistics kernel that run at a time (four per SIMD at almost every width)
@@ -1421,6 +1384,69 @@ GradientBlockPlan plan_gradient_blocks(int dvp, int D, int value_words_per_colum
   plan.lds_bytes =
       (plan.wave_floats + gradient_shared_fixed_floats(segment, value_words_per_column, 1)) *
       sizeof(float);
+  return plan;
+}
+
+// Waves of the gradient kernel that run at a time: what the registers of the form allow (the
+// form that walks pieces is compiled for fewer) and what the LDS of a block leaves room for.  The
+// grid has no more blocks than that: a block takes its first item by its number, and one that has
+// to wait for another to end would start the longest items last.
+constexpr size_t kLdsBytes = 160 * 1024;  // of a compute unit, handed out in kLdsGranule pieces
+constexpr size_t kLdsGranule = 1280;
+
+int64_t resident_gradient_waves(const GradientBlockPlan& block, int dvp, int symbol_tiles,
+                                bool pieces) {
+  const int by_registers = 4 * gradient_waves((dvp + 15) / 16, symbol_tiles, pieces);
+  const size_t lds = (block.lds_bytes + kLdsGranule - 1) / kLdsGranule * kLdsGranule;
+  const int by_lds = block.waves * static_cast<int>(kLdsBytes / std::max(lds, kLdsGranule));
+  return static_cast<int64_t>(device_simds() / 4) * std::max(block.waves, std::min(by_registers, by_lds));
+}
+
+// How the gradient kernel runs a problem (one slice of its value dimensions): the form of its
+// blocks, whether and how bands are cut into pieces that different waves walk, and the waves that
+// run at a time.  Bands are cut only with single-wave blocks, and only where whole ones would
+// leave resident waves idle (a band is as long as its diagonal, so the kernel would last as long
+// as its longest one).  A piece is a whole number of staged segments; piece_rows_for says how long.
+// The waves are those of the form that walks pieces: counted as the whole-band form's, three per
+// SIMD instead of two, 2 x 1024 tokens x 64 heads ran in one and a half rounds of 352-row pieces,
+// 270 us, now in one of 512-row pieces, 210.
+struct GradientPlan {
+  GradientBlockPlan block;
+  int piece_rows;   // 0: whole bands
+  int max_pieces;   // work items per band
+  int64_t waves;
+};
+
+GradientPlan plan_gradients(const Layout& L, int dvp, int value_words_per_column, int grad_pitch) {
+  const int64_t units = static_cast<int64_t>(L.slots) * L.H;
+  const int symbol_tiles = L.D > 16 ? 2 : 1;
+  GradientPlan plan;
+  plan.block = plan_gradient_blocks(dvp, L.D, value_words_per_column, grad_pitch, units);
+  plan.piece_rows = 0;
+  plan.max_pieces = 1;
+  plan.waves = resident_gradient_waves(plan.block, dvp, symbol_tiles, false);
+  if (plan.block.waves != 1) return plan;
+  const int64_t piece_waves = resident_gradient_waves(plan.block, dvp, symbol_tiles, true);
+  const int longest = L.varlen ? L.N : L.T;
+  int rows = 0;
+  const int forced_rows = g_gradient_piece_rows.load(std::memory_order_relaxed);
+  if (forced_rows > 0) {
+    rows = (std::max(forced_rows, 2 * kPieceAlign) + kPieceAlign - 1) / kPieceAlign * kPieceAlign;
+    if (longest - 1 <= rows) rows = 0;
+  } else if (forced_rows == 0 && g_gradient_block_waves.load(std::memory_order_relaxed) != 2 &&
+             units < 2 * piece_waves) {
+    // (a packed batch is cut on the device, by its actual lengths; here it counts as equal
+    // sequences)
+    const int64_t rows_in_all =
+        L.varlen ? static_cast<int64_t>(L.H) * L.S * band_steps_total(L.N / std::max(L.S, 1))
+                 : band_rows_at_most(L);
+    rows = piece_rows_for(rows_in_all, units, longest, piece_waves, kPieceRowsMin, kPieceAlign);
+  }
+  const int pieces = pieces_of_band(rows, longest);
+  if (rows <= 0 || pieces < 2 || units * pieces > INT32_MAX) return plan;
+  plan.piece_rows = rows;
+  plan.max_pieces = pieces;
+  plan.waves = piece_waves;
   return plan;
 }
 
@@ -1790,18 +1816,24 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
                            static_cast<int64_t>(max_segments > 0 ? max_groups + w.segment_group : 0) *
                                2 * kWave;
   const int64_t units = static_cast<int64_t>(v.L.slots) * v.L.H;
-  // resident waves of the gradient kernel (an even number: its blocks hold one or two waves)
-  const int64_t resident_cap = resident_gradient_waves((dvp + 15) / 16, v.L.D > 16 ? 2 : 1);
   // a piece per kPieceRowsMin rows or per resident wave's share, whichever is fewer, and one
   // more per band (the last piece of a band is a short one)
   w.stats_items_most =
       2 * units + std::min(band_rows_at_most(v.L) / kPieceRowsMin, 2 * resident_stats_waves());
-  // (work items at most: whole bands, or pieces of at least kPieceRowsMin rows)
-  const PiecePlan pieces = plan_band_pieces(v.L, resident_cap);
-  const int64_t items = pieces.max_pieces > 1 || v.L.varlen
-      ? units + band_rows_at_most(v.L) / kPieceRowsMin : units;
-  w.resident_blocks =
-      static_cast<int>(std::min<int64_t>((items + 1) & ~int64_t(1), resident_cap));
+  // Waves of the gradient kernel that run at a time (an even number: its blocks hold one or two),
+  // no more than there are work items: whole bands, or pieces of at least kPieceRowsMin rows.  The
+  // last slice of the value dimensions may be narrower and run differently.
+  w.resident_blocks = 2;
+  for (const int width : {slice_width, v.L.Dv % kValueSlice}) {
+    if (width == 0) continue;
+    const int slice_dvp = padded_value_width(width);
+    const GradientPlan plan = plan_gradients(v.L, slice_dvp, value_words(width),
+                                             grad_term_pitch(v.grad_terms, slice_dvp));
+    const int64_t items = plan.max_pieces > 1 || v.L.varlen
+        ? units + band_rows_at_most(v.L) / kPieceRowsMin : units;
+    w.resident_blocks = std::max(
+        w.resident_blocks, static_cast<int>(std::min((items + 1) & ~int64_t(1), plan.waves)));
+  }
   // keep the scratch pool below 2 GiB by running fewer resident blocks for huge windows
   const int64_t budget_floats = (int64_t(1) << 31) / 4;
   while (w.resident_blocks > 64 &&
@@ -2017,26 +2049,22 @@ int launch_vjp_passes(int nvw, int dvp, int symbol_tiles, bool dropout, const Vj
     stage_end(kStageRowMax, stream);
     if (status != 0) return status;
   }
-  const GradientBlockPlan plan = plan_gradient_blocks(dvp, P.L.D, nvw, P.grad_pitch, P.total_units);
+  const GradientPlan gradients = plan_gradients(P.L, dvp, nvw, P.grad_pitch);
+  const GradientBlockPlan& plan = gradients.block;
   Q.wave_lds_floats = static_cast<int>(plan.wave_floats);
   Q.exchange_tile_floats = static_cast<int>(plan.tile_floats);
   Q.row_queue = plan.row_queue ? 1 : 0;
-  Q.piece_rows = 0;
-  const int64_t resident = resident_gradient_waves((dvp + 15) / 16, symbol_tiles);
-  if (plan.waves == 1) {
-    const PiecePlan pieces = plan_band_pieces(P.L, resident);
-    Q.piece_rows = pieces.piece_rows;
-    if (!varlen && Q.piece_rows > 0) {
-      Q.items = static_cast<int>(pieces_of_sequence(P.L.T, Q.piece_rows) * P.L.B * P.L.H);
-    }
+  Q.piece_rows = gradients.piece_rows;
+  if (!varlen && Q.piece_rows > 0) {
+    Q.items = static_cast<int>(pieces_of_sequence(P.L.T, Q.piece_rows) * P.L.B * P.L.H);
   }
   Q.gradient_pieces = Q.piece_rows > 0 ? 1 : 0;
   stage_begin(kStageRowStats, stream);
   {
     int64_t blocks = varlen ? w.stats_items_most : units;
     if (!varlen) {
-      Q.stats_piece_rows = piece_rows_for(band_rows_at_most(P.L), P.L.T, resident_stats_waves(),
-                                          kPieceRowsMin, kChunk);
+      Q.stats_piece_rows = piece_rows_for(band_rows_at_most(P.L), units, P.L.T,
+                                          resident_stats_waves(), kPieceRowsMin, kChunk);
       if (Q.stats_piece_rows > 0) {
         blocks = pieces_of_sequence(P.L.T, Q.stats_piece_rows) * P.L.B * P.L.H;
       }
@@ -2052,12 +2080,13 @@ int launch_vjp_passes(int nvw, int dvp, int symbol_tiles, bool dropout, const Vj
                        stream, P.stats, rows, P.null_logit);
   }
   stage_end(kStageRowStats, stream);
-  const unsigned blocks = static_cast<unsigned>(std::max(1, w.resident_blocks / plan.waves));
+  const unsigned blocks = static_cast<unsigned>(
+      std::max<int64_t>(1, std::min<int64_t>(w.resident_blocks, gradients.waves) / plan.waves));
   const int form = plan.waves == 2 ? kGradientFormTwoWaves
                                    : Q.piece_rows > 0 ? kGradientFormPieces : kGradientFormOneWave;
   stage_begin(kStageGradients, stream);
   // both forms of the kernel (see its TERMS): the one that does not apply returns at once
-  Q.single_form = band_rows_at_most(P.L) <= kSingleFormRows * resident ? 1 : 0;
+  Q.single_form = band_rows_at_most(P.L) <= kSingleFormRows * gradients.waves ? 1 : 0;
   for (int terms = Q.single_form ? 3 : 2; terms <= 3 && status == 0; ++terms) {
     status = launch_band_kernel(kernels[vjp_kernel_slot_gradients(varlen, dropout, form, terms)],
                                 blocks, kWave * plan.waves, plan.lds_bytes, stream, Q);
@@ -2083,11 +2112,13 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
   Layout L = view.L;
   const VjpWorkspace w = carve_vjp(view, dropout_p > 0.0f);
   {
-    const int dvp = padded_value_width(std::min(L.Dv, kValueSlice));
-    const int64_t resident = resident_gradient_waves((dvp + 15) / 16, L.D > 16 ? 2 : 1);
+    const int width = std::min(L.Dv, kValueSlice);
+    const int dvp = padded_value_width(width);
+    const GradientPlan plan = plan_gradients(L, dvp, value_words(width),
+                                             grad_term_pitch(view.grad_terms, dvp));
     const int forced = g_gradient_piece_rows.load(std::memory_order_relaxed);
-    const PieceLimits limits{resident, resident_stats_waves(),
-                             forced > 0 ? plan_band_pieces(L, resident).piece_rows : forced,
+    const PieceLimits limits{std::min<int64_t>(plan.waves, w.resident_blocks), resident_stats_waves(),
+                             forced > 0 ? plan.piece_rows : forced,
                              w.stats_items_most, at<int32_t>(workspace, w.gradient_prefix),
                              at<int32_t>(workspace, w.stats_prefix)};
     launch_prepare_sequences(p, L, workspace, w.seq_start, w.seq_len, w.block_prefix, w.header,
@@ -3724,14 +3755,8 @@ int rosa_hip_gradient_piece_plan(const rosa_problem* problem, int* piece_rows, i
   if (status != 0) return status;
   const int slice_width = std::min(view.L.Dv, kValueSlice);
   const int dvp = padded_value_width(slice_width);
-  const int symbol_tiles = view.L.D > 16 ? 2 : 1;
-  const int64_t units = static_cast<int64_t>(view.L.slots) * view.L.H;
-  const GradientBlockPlan blocks = plan_gradient_blocks(
-      dvp, view.L.D, value_words(slice_width), grad_term_pitch(view.grad_terms, dvp), units);
-  PiecePlan plan{0, 1};
-  if (blocks.waves == 1) {
-    plan = plan_band_pieces(view.L, resident_gradient_waves((dvp + 15) / 16, symbol_tiles));
-  }
+  const GradientPlan plan = plan_gradients(view.L, dvp, value_words(slice_width),
+                                           grad_term_pitch(view.grad_terms, dvp));
   if (piece_rows != nullptr) *piece_rows = plan.piece_rows;
   if (pieces != nullptr) *pieces = plan.max_pieces;
   return 0;

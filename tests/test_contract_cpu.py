@@ -341,6 +341,47 @@ def test_gradient_launch_plan_follows_the_shape():
     assert plan(torch.float32, (2, 4096, 64), 8, 16, 8, 128) == metric
 
 
+@pytest.mark.parametrize("dtype,B,T,H,D,Hv,Dv,W,p,waves", [
+    (torch.float32, 2, 1024, 64, 8, 16, 8, 128, 0.1, 2048),    # narrow tile: three waves whole, two cut
+    (torch.bfloat16, 2, 1024, 32, 8, 32, 64, 64, 0.0, 1024),   # width 64: two waves whole, one cut
+    (torch.float32, 1, 1500, 16, 8, 16, 64, 32, 0.1, 1024),
+    (torch.float32, 1, 4096, 8, 8, 8, 8, 64, 0.0, 2048),
+    (torch.float16, 1, 2048, 16, 20, 16, 32, 64, 0.0, 2048),
+    (torch.bfloat16, 1, 900, 3, 8, 3, 16, 16, 0.0, 2048),
+])
+def test_pieces_of_bands_are_planned_for_the_waves_of_the_form_that_walks_them(dtype, B, T, H, D, Hv, Dv,
+                                                                               W, p, waves):
+    """Host arithmetic on 1024 SIMDs.  The form that walks pieces has `waves` resident waves (its
+    registers, in the resource report, allow no more), the scratch is laid out for no more, and
+    full pieces come to one round: as many as there are waves, beyond the halves of bands that
+    have a wave each."""
+
+    query, value = torch.empty(B, T, H, D, dtype=dtype), torch.empty(B, T, Hv, Dv, dtype=dtype)
+    plan = cabi.gradient_block_plan(query, value, W)
+    rows = plan["piece_rows"]
+    assert plan["waves"] == 1 and rows > 0 and rows % 32 == 0
+    bands = [T - 1 - 64 * j for j in range((T - 2) // 64 + 1)] * (B * H)
+    full = sum(n // rows for n in bands)
+    assert full <= waves
+    if len(bands) > waves // 2 and rows >= T // 2:
+        assert len(bands) <= waves
+    else:  # and no coarser than that takes: a tenth above the share of a wave, in whole segments
+        assert rows <= max(32, 1.1 * sum(bands) / waves + 32)
+    # one ring of six bytes per lane and window row for every resident wave, by two windows
+    size = lambda window: cabi.load().rosa_hip_vjp_workspace_bytes(
+        ctypes.byref(cabi.make_problem(query, value, window)), 7, 1.0, int(p > 0))
+    rings = round((size(W + 8) - size(W)) / (8 * 64 * 6))
+    assert rings <= waves
+    from rosa_soft_amd import _build
+    if os.path.exists(_build.RESOURCE_REPORT):
+        import json
+        width = 8 if Dv <= 8 else 16 if Dv <= 16 else 32 if Dv <= 32 else 64
+        form = f"vjp_gradients_kernelILi{1 + (Dv > 32)}ELi{width}ELi{1 + (D > 16)}ELb0ELb{int(p > 0)}ELi1ELi3ELb1E"
+        with open(_build.RESOURCE_REPORT) as handle:
+            found = [use for name, use in json.load(handle).items() if form in name]
+        assert len(found) == 1 and 1024 * found[0]["waves_per_simd"] == waves
+
+
 def test_no_kernel_of_the_last_build_spills_or_uses_scratch():
     """The build records what the compiler reported per kernel.  Spilled vector registers and
     scratch memory are performance faults of the backward kernels (a reload waits behind
