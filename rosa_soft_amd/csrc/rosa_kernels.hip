@@ -2061,17 +2061,25 @@ int launch_vjp_passes(int nvw, int dvp, int symbol_tiles, bool dropout, const Vj
   Q.gradient_pieces = Q.piece_rows > 0 ? 1 : 0;
   stage_begin(kStageRowStats, stream);
   {
-    int64_t blocks = varlen ? w.stats_items_most : units;
-    if (!varlen) {
-      Q.stats_piece_rows = piece_rows_for(band_rows_at_most(P.L), units, P.L.T,
-                                          resident_stats_waves(), kPieceRowsMin, kChunk);
+    // Whole bands or pieces: by the plan, for a packed batch, whose lengths only the device has,
+    // by the number of bands (with two per wave or more the longest one no longer decides).
+    const int64_t waves = resident_stats_waves();
+    int64_t blocks = units;
+    bool in_pieces = Q.gradient_pieces != 0;  // the records that pieces of the gradient pass need
+    if (varlen) {
+      in_pieces = in_pieces || units < 2 * waves;
+      if (in_pieces) blocks = w.stats_items_most;
+    } else {
+      Q.stats_piece_rows =
+          piece_rows_for(band_rows_at_most(P.L), units, P.L.T, waves, kPieceRowsMin, kChunk);
       if (Q.stats_piece_rows > 0) {
+        in_pieces = true;
         blocks = pieces_of_sequence(P.L.T, Q.stats_piece_rows) * P.L.B * P.L.H;
       }
     }
-    status = launch_band_kernel(row_kernels[vjp_kernel_slot_row_stats(varlen, dropout)],
-                                static_cast<unsigned>(blocks), kWave,
-                                row_stats_dynamic_lds(P.grad_pitch), stream, Q);
+    status = launch_band_kernel(
+        row_kernels[vjp_kernel_slot_row_stats(varlen, dropout, in_pieces ? 1 : 0)],
+        static_cast<unsigned>(blocks), kWave, row_stats_dynamic_lds(P.grad_pitch), stream, Q);
     if (status != 0) return status;
   }
   if (Q.gradient_pieces == 0) {

@@ -704,22 +704,29 @@ __device__ __forceinline__ v4f tile_row_sums(const float* tile_rows, int pitch, 
   return mfma_16x16x4(partial, 1.0f, v4f{0.0f, 0.0f, 0.0f, 0.0f});
 }
 
-// Waves per SIMD the row-statistics kernel is compiled for (no variant spills at these; the
-// widest tile with dropout is one register short of four).  Its LDS allows four with 16-bit
-// inputs at every width.
-constexpr int row_stats_waves(int dvp, bool dropout) { return dvp > 32 && dropout ? 3 : 4; }
+// Waves per SIMD the row-statistics kernel is compiled for (no variant spills at these; the form
+// that walks pieces is four registers short of four at the widest tile with dropout).  Its LDS
+// allows four with 16-bit inputs at every width.
+constexpr int row_stats_waves(int dvp, bool dropout, bool pieces) {
+  return dvp > 32 && dropout && pieces ? 3 : 4;
+}
 
 constexpr float kLongMatchEvidence = 6.0f;
 
 // Row-statistics pass: denominator and expected dropped utility of every row.
+// PIECES: bands are cut into pieces, and the gradient pass is told how soon gates multiply to
+// nothing; compiled apart.  In one kernel the piece's bounds and the mismatches of a chunk live
+// through the chunk loop of whole bands too, which cost large problems 1 to 2 % and width 64
+// with dropout its fourth wave per SIMD (132 registers for 127: 2.22 ms for 1.97 at 4 x 4096
+// tokens x 32 heads).
 // Rows are processed 16 at a time without any branch in between.  A chunk leaves
 // its route weights and its dropped weighted utilities as two [row][lane] tiles
 // in LDS; their row sums are formed on the matrix cores and leave in one atomic
 // each from 16 lanes; every lane keeps its 16 dropout decisions of the chunk as bits and
 // stores them with the chunk's checkpoint for the gradient pass.
-template <int NVW, int DVP, bool VARLEN, bool DROPOUT>
+template <int NVW, int DVP, bool VARLEN, bool DROPOUT, bool PIECES>
 __global__ __launch_bounds__(kWave)
-__attribute__((amdgpu_waves_per_eu(row_stats_waves(DVP, DROPOUT))))
+__attribute__((amdgpu_waves_per_eu(row_stats_waves(DVP, DROPOUT, PIECES))))
 void vjp_row_stats_kernel(VjpParams P) {
   // rows staged in LDS at a time: one chunk, loaded a chunk ahead.  With the half-height
   // weight tile below a block's LDS stays under 10 KB, which lets four waves share a SIMD
@@ -742,14 +749,16 @@ void vjp_row_stats_kernel(VjpParams P) {
   float* const discard = weights;
   // (the host sizes the grid of a packed batch before it knows the lengths: blocks beyond the
   // items it turns out to have return at once)
-  const int piece_rows = VARLEN ? table_value<true>(P.header[kHeaderStatsPieces]) : P.stats_piece_rows;
-  int piece = 0;
+  int piece_rows = 0, piece = 0;
+  if constexpr (PIECES) {
+    piece_rows = VARLEN ? table_value<true>(P.header[kHeaderStatsPieces]) : P.stats_piece_rows;
+  }
   Unit u;
-  if (piece_rows > 0) {
+  if (PIECES && piece_rows > 0) {
     if (VARLEN && static_cast<int>(blockIdx.x) >= P.header[kHeaderStatsPieces + 1]) return;
     u = decode_piece<VARLEN>(P.L, P.stats_prefix, piece_rows, blockIdx.x, piece);
   } else {
-    if (VARLEN && static_cast<int>(blockIdx.x) >= P.total_units) return;
+    if (PIECES && VARLEN && static_cast<int>(blockIdx.x) >= P.total_units) return;
     u = decode_unit<VARLEN>(P.L, blockIdx.x);
   }
   if (!u.valid) return;
@@ -757,9 +766,9 @@ void vjp_row_stats_kernel(VjpParams P) {
   int hv;
   if (!make_view<NVW, VARLEN>(P, u, view, hv)) return;
   // rows [row_begin, row_end) of the band are this work item's
-  const int row_begin = piece * piece_rows;
-  if (row_begin >= view.steps) return;
-  const int row_end = piece_rows > 0 ? min(view.steps, row_begin + piece_rows) : view.steps;
+  const int row_begin = PIECES ? piece * piece_rows : 0;
+  if (PIECES && row_begin >= view.steps) return;
+  const int row_end = PIECES && piece_rows > 0 ? min(view.steps, row_begin + piece_rows) : view.steps;
   const int lane = threadIdx.x;
   const int W = P.L.W;
   DropoutKey key;
@@ -774,8 +783,14 @@ void vjp_row_stats_kernel(VjpParams P) {
   }
   const float logit_gain = in_vector_register(P.logit_gain);
   Band<NVW> band;
-  enter_piece<NVW>(band, view, row_begin, lane, W, P.gate_log2);
-  band.window += kCountBias;  // forward_step<..., BIASED>
+  if constexpr (PIECES) {
+    enter_piece<NVW>(band, view, row_begin, lane, W, P.gate_log2);
+    band.window += kCountBias;  // forward_step<..., BIASED>
+  } else {
+    band.evidence = 0.0f;
+    band.window = kCountBias;
+    load_sliding<NVW>(band, view, 0, lane, W);
+  }
   const bool needs_utility = (P.gradient_mask & (ROSA_GRAD_QUERY | ROSA_GRAD_KEY)) != 0;
   uint32_t route_hash = route_hash_of(row_begin - lane);
   const int last_step = view.steps - 1;
@@ -866,7 +881,7 @@ void vjp_row_stats_kernel(VjpParams P) {
   int pending_window = 0;
   uint32_t pending_kept = 0u;
   int pending_first = -1, pending_rows = 0;
-  int pending_decay = 0;
+  [[maybe_unused]] int pending_decay = 0;
   const auto flush_outputs = [&]() {
     if (pending_first < 0) return;
     // lanes 0..3 of every 16-lane group write the four rows of their group
@@ -881,8 +896,10 @@ void vjp_row_stats_kernel(VjpParams P) {
       float* slot =
           view.checkpoints + static_cast<int64_t>(pending_first / kChunk) * view.record_floats;
       reinterpret_cast<uint16_t*>(slot + kWave)[lane] = static_cast<uint16_t>(pending_window);
-      if (P.gradient_pieces != 0 && lane == 63) {
-        view.chunk_decay[pending_first / kChunk] = static_cast<uint16_t>(pending_decay);
+      if constexpr (PIECES) {
+        if (P.gradient_pieces != 0 && lane == 63) {
+          view.chunk_decay[pending_first / kChunk] = static_cast<uint16_t>(pending_decay);
+        }
       }
       if constexpr (DROPOUT) {
         // the gradient pass reads the decisions back instead of hashing again
@@ -940,7 +957,8 @@ void vjp_row_stats_kernel(VjpParams P) {
         wave_lds_fence();
       }
       uint32_t kept_bits = 0u;  // bit r: this lane's pair of row r is kept
-      uint32_t entering = 0u;   // mismatching bits of this lane's pairs of the chunk
+      // mismatching bits of this lane's pairs of the chunk (of quiet chunks, or with PIECES)
+      uint32_t entering = 0u;
       v4f first_weight_sums;    // of rows 0 .. 7
       // compiled twice: once every lane is past its window fill no masking is needed
       auto run_chunk = [&](auto steady_tag, auto quiet_tag) {
@@ -1068,7 +1086,7 @@ void vjp_row_stats_kernel(VjpParams P) {
             s.active = true;
           } else {
             s = forward_step<NVW, STEADY, false, true>(band, symbols, i, lane, W, P.gate_log2);
-            entering += static_cast<uint32_t>(s.mismatches);
+            if constexpr (PIECES) entering += static_cast<uint32_t>(s.mismatches);
             peak_overflow = fmaxf(peak_overflow, s.overflow);
           }
           // (outside quiet chunks the root is formed exactly as the gradient pass forms it:
@@ -1142,7 +1160,7 @@ void vjp_row_stats_kernel(VjpParams P) {
       if ((noisy || long_match) && lane == 0) P.work_counter[3] = 1;
       // (a chunk of the band's first rows, where lanes have no pair yet, or with rows beyond the
       // band's end counts for nothing)
-      if (P.gradient_pieces != 0) {
+      if (PIECES && P.gradient_pieces != 0) {
         pending_decay = chunk_first >= kWave && rows_here == kChunk
                             ? wave_min_lane63(min(entering, 0xffffu)) : 0;
       }
@@ -2374,10 +2392,12 @@ constexpr int kGradientFormOneWave = 0;   // single-wave blocks, whole bands
 constexpr int kGradientFormTwoWaves = 1;  // two-wave blocks
 constexpr int kGradientFormPieces = 2;    // single-wave blocks, bands cut into pieces
 constexpr int vjp_kernel_slot_row_max(int varlen) { return varlen; }
-constexpr int vjp_kernel_slot_row_stats(int varlen, int dropout) { return 2 + 2 * varlen + dropout; }
-constexpr int vjp_kernel_slot_gradients(int varlen, int dropout, int form, int terms) {
-  return 6 + ((2 * varlen + dropout) * 3 + form) * 2 + (terms - 2);
+constexpr int vjp_kernel_slot_row_stats(int varlen, int dropout, int pieces) {
+  return 2 + (2 * varlen + dropout) * 2 + pieces;
 }
-constexpr int kVjpKernelSlots = 6 + 4 * 3 * 2;
+constexpr int vjp_kernel_slot_gradients(int varlen, int dropout, int form, int terms) {
+  return 10 + ((2 * varlen + dropout) * 3 + form) * 2 + (terms - 2);
+}
+constexpr int kVjpKernelSlots = 10 + 4 * 3 * 2;
 
 }  // namespace

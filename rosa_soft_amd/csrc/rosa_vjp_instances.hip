@@ -41,8 +41,10 @@ void fill_layout(const void** table) {
   if constexpr (DT == 1) {
     // the row kernels do not depend on the symbol tiles: they live in the one-tile family
     table[vjp_kernel_slot_row_max(v)] = address_of(vjp_row_max_kernel<NVW, VARLEN>);
-    table[vjp_kernel_slot_row_stats(v, d)] =
-        address_of(vjp_row_stats_kernel<NVW, DVP, VARLEN, DROPOUT>);
+    table[vjp_kernel_slot_row_stats(v, d, 0)] =
+        address_of(vjp_row_stats_kernel<NVW, DVP, VARLEN, DROPOUT, false>);
+    table[vjp_kernel_slot_row_stats(v, d, 1)] =
+        address_of(vjp_row_stats_kernel<NVW, DVP, VARLEN, DROPOUT, true>);
   }
   table[vjp_kernel_slot_gradients(v, d, kGradientFormOneWave, 2)] =
       address_of(vjp_gradients_kernel<NVW, DVP, DT, VARLEN, DROPOUT, 1, 2, false>);

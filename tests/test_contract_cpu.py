@@ -425,6 +425,32 @@ def test_no_kernel_of_the_last_build_spills_or_uses_scratch():
             assert registers <= budget[3 if wide_with_dropout else 4], (name, registers)
 
 
+def test_whole_bands_of_the_row_statistics_pass_keep_four_waves_per_simd():
+    """The row-statistics kernel has a form for whole bands, which large problems run, without the
+    bounds and mismatch counts of pieces: it fits four waves per SIMD (128 registers) at every
+    width, with dropout too, and needs fewer registers than the form that walks pieces."""
+
+    from rosa_soft_amd import _build
+
+    if not os.path.exists(_build.RESOURCE_REPORT):
+        pytest.skip("the HIP library is not built")
+    import json
+
+    with open(_build.RESOURCE_REPORT) as handle:
+        report = json.load(handle)
+    found = {}
+    for name, use in report.items():
+        match = re.search(r"vjp_row_stats_kernelILi(\d)ELi(\d+)ELb(\d)ELb(\d)ELb(\d)EEE", name)
+        if match:
+            *tile, pieces = (int(x) for x in match.groups())
+            found[tuple(tile), pieces] = use
+    assert len(found) == 4 * 2 * 2 * 2
+    for (tile, pieces), use in found.items():
+        if not pieces:
+            assert use["waves_per_simd"] == 4 and use["vgprs"] <= 128, (tile, use)
+            assert use["vgprs"] < found[tile, 1]["vgprs"], tile
+
+
 def test_no_product_module_imports_the_oracle():
     package = os.path.join(ROOT, "rosa_soft_amd")
     for name in os.listdir(package):
