@@ -1313,6 +1313,31 @@ int device_simds() {
   return simds;
 }
 
+constexpr size_t kLdsBytes = 160 * 1024;  // of a compute unit, handed out in kLdsGranule pieces
+constexpr size_t kLdsGranule = 1280;
+
+// waves of a band kernel that run at a time: `per_simd` by its registers, and by the LDS of its
+// blocks of `block_waves` waves
+int64_t resident_waves(int per_simd, int block_waves, size_t block_lds) {
+  const size_t lds = (std::max<size_t>(block_lds, 1) + kLdsGranule - 1) / kLdsGranule * kLdsGranule;
+  const int by_lds = block_waves * static_cast<int>(kLdsBytes / lds);
+  return static_cast<int64_t>(device_simds() / 4) *
+         std::max(block_waves, std::min(4 * per_simd, by_lds));
+}
+
+// dynamic LDS of a block of the row-statistics kernel: the bfloat16 terms of its grad_output
+// rows as the launch needs them
+size_t row_stats_dynamic_lds(int grad_pitch) {
+  constexpr int kBlockRows = kChunk;  // as in the kernel
+  return sizeof(uint16_t) * kBlockRows * static_cast<size_t>(grad_pitch + 8);
+}
+
+// waves of the row-statistics kernel that run at a time, in the form that walks pieces
+int64_t resident_stats_waves(int dvp, bool dropout, int grad_pitch) {
+  return resident_waves(row_stats_waves(dvp, dropout, true), 1,
+                        row_stats_static_lds(dvp > 32 ? 2 : 1) + row_stats_dynamic_lds(grad_pitch));
+}
+
 // blocks of the gradient kernel that are resident at two waves per SIMD
 int max_resident_blocks() { return 2 * device_simds(); }
 
@@ -1333,9 +1358,6 @@ int64_t band_rows_at_most(const Layout& L) {
   return L.varlen ? static_cast<int64_t>(L.H) * band_steps_total(L.N)
                   : static_cast<int64_t>(L.B) * L.H * band_steps_total(L.T);
 }
-
-// waves of the row-statistics kernel that run at a time (four per SIMD at almost every width)
-int64_t resident_stats_waves() { return 4 * static_cast<int64_t>(device_simds()); }
 
 // Up to this many rows per resident wave the gradient pass runs as its three-term form alone,
 // which serves every input: below it the launch that returns at once would cost more than
@@ -1391,15 +1413,10 @@ GradientBlockPlan plan_gradient_blocks(int dvp, int D, int value_words_per_colum
 // form that walks pieces is compiled for fewer) and what the LDS of a block leaves room for.  The
 // grid has no more blocks than that: a block takes its first item by its number, and one that has
 // to wait for another to end would start the longest items last.
-constexpr size_t kLdsBytes = 160 * 1024;  // of a compute unit, handed out in kLdsGranule pieces
-constexpr size_t kLdsGranule = 1280;
-
 int64_t resident_gradient_waves(const GradientBlockPlan& block, int dvp, int symbol_tiles,
                                 bool pieces) {
-  const int by_registers = 4 * gradient_waves((dvp + 15) / 16, symbol_tiles, pieces);
-  const size_t lds = (block.lds_bytes + kLdsGranule - 1) / kLdsGranule * kLdsGranule;
-  const int by_lds = block.waves * static_cast<int>(kLdsBytes / std::max(lds, kLdsGranule));
-  return static_cast<int64_t>(device_simds() / 4) * std::max(block.waves, std::min(by_registers, by_lds));
+  return resident_waves(gradient_waves((dvp + 15) / 16, symbol_tiles, pieces), block.waves,
+                        block.lds_bytes);
 }
 
 // How the gradient kernel runs a problem (one slice of its value dimensions): the form of its
@@ -1733,6 +1750,7 @@ struct VjpWorkspace {
   size_t sums_query, sums_key, sums_value;  // head-major accumulators (rows of <= 8 floats)
   bool symbols_by_head, values_by_head;
   size_t checkpoints, chunk_decay;
+  int64_t stats_waves;          // of the row-statistics pass that run at a time, in pieces
   int64_t stats_items_most;     // work items the row-statistics grid of a packed batch has room for
   size_t gradient_prefix, stats_prefix;
   int64_t checkpoint_capacity;  // chunk records that fit in the workspace (0: none kept)
@@ -1818,8 +1836,9 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
   const int64_t units = static_cast<int64_t>(v.L.slots) * v.L.H;
   // a piece per kPieceRowsMin rows or per resident wave's share, whichever is fewer, and one
   // more per band (the last piece of a band is a short one)
+  w.stats_waves = resident_stats_waves(dvp, dropout, grad_term_pitch(v.grad_terms, dvp));
   w.stats_items_most =
-      2 * units + std::min(band_rows_at_most(v.L) / kPieceRowsMin, 2 * resident_stats_waves());
+      2 * units + std::min(band_rows_at_most(v.L) / kPieceRowsMin, 2 * w.stats_waves);
   // Waves of the gradient kernel that run at a time (an even number: its blocks hold one or two),
   // no more than there are work items: whole bands, or pieces of at least kPieceRowsMin rows.  The
   // last slice of the value dimensions may be narrower and run differently.
@@ -1991,12 +2010,6 @@ int run_forward(const rosa_problem* p, const ProblemView& view, const void* quer
   return 0;
 }
 
-// bytes of the staged grad_output rows of a block of the row-statistics kernel
-size_t row_stats_dynamic_lds(int grad_pitch) {
-  constexpr int kBlockRows = kChunk;  // as in the kernel
-  return sizeof(uint16_t) * kBlockRows * static_cast<size_t>(grad_pitch + 8);
-}
-
 // The band kernels are compiled in translation units of their own, one per tile family
 // (sign words per value column, padded value width, symbol tiles); each exports its table
 // of kernel addresses (see vjp_kernel_slot in rosa_vjp_bands.hpp).
@@ -2063,7 +2076,7 @@ int launch_vjp_passes(int nvw, int dvp, int symbol_tiles, bool dropout, const Vj
   {
     // Whole bands or pieces: by the plan, for a packed batch, whose lengths only the device has,
     // by the number of bands (with two per wave or more the longest one no longer decides).
-    const int64_t waves = resident_stats_waves();
+    const int64_t waves = resident_stats_waves(dvp, dropout, P.grad_pitch);
     int64_t blocks = units;
     bool in_pieces = Q.gradient_pieces != 0;  // the records that pieces of the gradient pass need
     if (varlen) {
@@ -2125,7 +2138,7 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
     const GradientPlan plan = plan_gradients(L, dvp, value_words(width),
                                              grad_term_pitch(view.grad_terms, dvp));
     const int forced = g_gradient_piece_rows.load(std::memory_order_relaxed);
-    const PieceLimits limits{std::min<int64_t>(plan.waves, w.resident_blocks), resident_stats_waves(),
+    const PieceLimits limits{std::min<int64_t>(plan.waves, w.resident_blocks), w.stats_waves,
                              forced > 0 ? plan.piece_rows : forced,
                              w.stats_items_most, at<int32_t>(workspace, w.gradient_prefix),
                              at<int32_t>(workspace, w.stats_prefix)};

@@ -711,6 +711,11 @@ constexpr int row_stats_waves(int dvp, bool dropout, bool pieces) {
   return dvp > 32 && dropout && pieces ? 3 : 4;
 }
 
+// bytes of static LDS of a block of the row-statistics kernel (asserted there)
+constexpr size_t row_stats_static_lds(int value_words_per_column) {
+  return 7168 + 320 * static_cast<size_t>(value_words_per_column);
+}
+
 constexpr float kLongMatchEvidence = 6.0f;
 
 // Row-statistics pass: denominator and expected dropped utility of every row.
@@ -746,6 +751,8 @@ void vjp_row_stats_kernel(VjpParams P) {
   // are formed it takes the elements of the edge tiles that belong to no lane
   constexpr int kWeightRows = kChunk / 2;
   __shared__ __attribute__((aligned(16))) float weights[kWeightRows * kWeightPitch];
+  static_assert(sizeof(rows) + sizeof(sign_table) + sizeof(value_columns) + sizeof(utilities) +
+                    sizeof(weights) == row_stats_static_lds(NVW), "static LDS of a block");
   float* const discard = weights;
   // (the host sizes the grid of a packed batch before it knows the lengths: blocks beyond the
   // items it turns out to have return at once)
