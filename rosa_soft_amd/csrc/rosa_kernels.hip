@@ -1432,6 +1432,8 @@ struct GradientPlan {
   int piece_rows;   // 0: whole bands
   int max_pieces;   // work items per band
   int64_t waves;
+  int64_t items;    // work items at most
+  int ring_rows;    // rows of a wave's ring
 };
 
 GradientPlan plan_gradients(const Layout& L, int dvp, int value_words_per_column, int grad_pitch) {
@@ -1442,9 +1444,11 @@ GradientPlan plan_gradients(const Layout& L, int dvp, int value_words_per_column
   plan.piece_rows = 0;
   plan.max_pieces = 1;
   plan.waves = resident_gradient_waves(plan.block, dvp, symbol_tiles, false);
+  const int longest = L.varlen ? L.N : L.T;
+  plan.items = units;
+  plan.ring_rows = L.W + 1;
   if (plan.block.waves != 1) return plan;
   const int64_t piece_waves = resident_gradient_waves(plan.block, dvp, symbol_tiles, true);
-  const int longest = L.varlen ? L.N : L.T;
   int rows = 0;
   const int forced_rows = g_gradient_piece_rows.load(std::memory_order_relaxed);
   if (forced_rows > 0) {
@@ -1464,6 +1468,20 @@ GradientPlan plan_gradients(const Layout& L, int dvp, int value_words_per_column
   plan.piece_rows = rows;
   plan.max_pieces = pieces;
   plan.waves = piece_waves;
+  // The work items, and the rows a piece walks: its own and a halo of whole chunks below it.  The
+  // lengths of a packed batch may ask for pieces of up to what one sequence of all tokens would.
+  int longest_piece = rows;
+  if (!L.varlen) {
+    plan.items = pieces_of_sequence(L.T, rows) * L.B * L.H;
+  } else if (forced_rows > 0) {
+    plan.items = units + band_rows_at_most(L) / rows;
+  } else {
+    plan.items = units + std::min(band_rows_at_most(L) / kPieceRowsMin, piece_waves);
+    longest_piece = piece_rows_for(band_rows_at_most(L), INT64_MAX, INT32_MAX, piece_waves,
+                                   kPieceRowsMin, kPieceAlign);
+  }
+  const int64_t halo = (static_cast<int64_t>(L.W) - 1 + kChunk - 1) / kChunk * kChunk;
+  plan.ring_rows = gradient_ring_rows(L.W, std::min<int64_t>(longest - 1, longest_piece + halo));
   return plan;
 }
 
@@ -1812,7 +1830,6 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
     cursor += align_up(sizeof(uint16_t) * static_cast<size_t>(w.checkpoint_capacity));
   }
   const int longest = v.L.varlen ? v.L.N : v.L.T;
-  w.ring_rows = std::min(v.L.W, longest) + 1;
   const int segment_rows = gradient_segment(dvp);
   // one fallback checkpoint per segment of the longest possible band, for a wave that finds
   // no records: never the case in a dense layout whose records fit (known here), decided on
@@ -1820,7 +1837,7 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
   // (nor in one whose window counts the records can always hold: see the launch)
   const bool may_run_without_records =
       v.L.varlen != 0 || w.checkpoint_capacity == 0 ||
-      (static_cast<int64_t>(w.ring_rows) * v.L.D > kRecordWindowMax);
+      ((static_cast<int64_t>(v.L.W) + 1) * v.L.D > kRecordWindowMax);
   const int max_segments =
       may_run_without_records ? (longest + segment_rows - 1) / segment_rows + 1 : 0;
   // two levels: a checkpoint per group of G segments and one per segment of a group, with G
@@ -1828,11 +1845,6 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
   w.segment_group = 4;
   while (w.segment_group * w.segment_group < max_segments) ++w.segment_group;
   const int max_groups = max_segments > 0 ? (max_segments + w.segment_group - 1) / w.segment_group : 0;
-  // (the ring holds a float and a bfloat16 per row and lane)
-  w.block_scratch_floats = static_cast<int64_t>(w.ring_rows) * (kWave + kWave / 2) +
-                           2 * kCheckpointChunksMax * kWave +
-                           static_cast<int64_t>(max_segments > 0 ? max_groups + w.segment_group : 0) *
-                               2 * kWave;
   const int64_t units = static_cast<int64_t>(v.L.slots) * v.L.H;
   // a piece per kPieceRowsMin rows or per resident wave's share, whichever is fewer, and one
   // more per band (the last piece of a band is a short one)
@@ -1840,19 +1852,24 @@ VjpWorkspace carve_vjp(const ProblemView& v, bool dropout) {
   w.stats_items_most =
       2 * units + std::min(band_rows_at_most(v.L) / kPieceRowsMin, 2 * w.stats_waves);
   // Waves of the gradient kernel that run at a time (an even number: its blocks hold one or two),
-  // no more than there are work items: whole bands, or pieces of at least kPieceRowsMin rows.  The
-  // last slice of the value dimensions may be narrower and run differently.
+  // no more than there are work items.  The last slice of the value dimensions may be narrower
+  // and run differently.
   w.resident_blocks = 2;
+  w.ring_rows = 1;
   for (const int width : {slice_width, v.L.Dv % kValueSlice}) {
     if (width == 0) continue;
     const int slice_dvp = padded_value_width(width);
     const GradientPlan plan = plan_gradients(v.L, slice_dvp, value_words(width),
                                              grad_term_pitch(v.grad_terms, slice_dvp));
-    const int64_t items = plan.max_pieces > 1 || v.L.varlen
-        ? units + band_rows_at_most(v.L) / kPieceRowsMin : units;
     w.resident_blocks = std::max(
-        w.resident_blocks, static_cast<int>(std::min((items + 1) & ~int64_t(1), plan.waves)));
+        w.resident_blocks, static_cast<int>(std::min((plan.items + 1) & ~int64_t(1), plan.waves)));
+    w.ring_rows = std::max(w.ring_rows, plan.ring_rows);
   }
+  // (the ring holds a float and a bfloat16 per row and lane; that of pieces a row that nobody reads)
+  w.block_scratch_floats = static_cast<int64_t>(w.ring_rows + 1) * (kWave + kWave / 2) +
+                           2 * kCheckpointChunksMax * kWave +
+                           static_cast<int64_t>(max_segments > 0 ? max_groups + w.segment_group : 0) *
+                               2 * kWave;
   // keep the scratch pool below 2 GiB by running fewer resident blocks for huge windows
   const int64_t budget_floats = (int64_t(1) << 31) / 4;
   while (w.resident_blocks > 64 &&
@@ -2068,6 +2085,8 @@ int launch_vjp_passes(int nvw, int dvp, int symbol_tiles, bool dropout, const Vj
   Q.exchange_tile_floats = static_cast<int>(plan.tile_floats);
   Q.row_queue = plan.row_queue ? 1 : 0;
   Q.piece_rows = gradients.piece_rows;
+  Q.ring_rows = gradients.ring_rows;
+  Q.ring_skip = (P.L.W + 1) % gradients.ring_rows;
   if (!varlen && Q.piece_rows > 0) {
     Q.items = static_cast<int>(pieces_of_sequence(P.L.T, Q.piece_rows) * P.L.B * P.L.H);
   }
@@ -2275,7 +2294,7 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
     // below the saturation value (otherwise, with a long window and a tiny mismatch_scale,
     // the gradient pass rebuilds the evidence itself).
     const bool windows_fit =
-        static_cast<int64_t>(w.ring_rows) * L.D <= kRecordWindowMax ||
+        (static_cast<int64_t>(L.W) + 1) * L.D <= kRecordWindowMax ||
         -std::log2(P.tail_threshold) / P.gate_log2 + kChunk * L.D + 2 <= kRecordWindowMax;
     P.checkpoints = (w.checkpoint_capacity > 0 && windows_fit) ? at<float>(workspace, w.checkpoints)
                                                               : nullptr;
@@ -2285,7 +2304,6 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
     P.block_scratch = at<float>(workspace, w.block_scratch);
     P.block_scratch_floats = w.block_scratch_floats;
     P.segment_group = w.segment_group;
-    P.ring_rows = w.ring_rows;
     P.chunk_decay = at<uint16_t>(workspace, w.chunk_decay);
     P.gradient_prefix = at<int32_t>(workspace, w.gradient_prefix);
     P.stats_prefix = at<int32_t>(workspace, w.stats_prefix);

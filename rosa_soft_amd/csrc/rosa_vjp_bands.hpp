@@ -47,7 +47,7 @@ struct VjpParams {
   float* block_scratch;         // per resident block: ring + segment checkpoints
   int64_t block_scratch_floats;
   int segment_group;            // segments per group of the fallback checkpoints (see carve_vjp)
-  int ring_rows;                // W + 1 clipped to the longest possible diagonal
+  int ring_rows;                // rows a ring holds: W + 1, or gradient_ring_rows for pieces
   int total_units;
   int wave_lds_floats;          // LDS floats each wave of a gradient block owns
   int exchange_tile_floats;     // LDS floats of an accumulator tile passed between waves
@@ -65,10 +65,21 @@ struct VjpParams {
   // overflow terms, and below 2^-150 nothing is left of a float32.  (A bound relative to the
   // carry, 2^-34 of it and the like, is not enough: rows of grad_output may differ by any factor.)
   float halo_decay;
+  int ring_skip;                // (pieces) (W + 1) mod ring_rows
   int single_form;              // only the three-term form of the gradient kernel is launched
   uint16_t* chunk_decay;        // per chunk record: fewest mismatching bits any diagonal of the band
                                 // meets in the chunk's 16 rows
 };
+
+// Rows of the ring that holds the overflow terms of a walk upwards over at most `walked` rows: the
+// term of a row leaves the window sum W + 1 rows above it, so the last W + 1 rows' terms are
+// needed at a time, and those of the walk's last W + 1 rows not at all.  Pieces therefore take
+// little more than their own rows, and next to none where the window is near the sequence.  (Whole
+// bands keep W + 1 rows: one slot per row, and no more of them than the chip has waves.)
+constexpr int gradient_ring_rows(int window, int64_t walked) {
+  const int64_t stored = walked - window - 1;
+  return static_cast<int>(stored < 1 ? 1 : stored > window + 1 ? window + 1 : stored);
+}
 
 // header words that hold the piece plan of a packed batch
 constexpr int kHeaderGradientPieces = 5;  // rows, then work items in all
@@ -1188,9 +1199,9 @@ void vjp_row_stats_kernel(VjpParams P) {
 // therefore rebuilt from checkpoints: one cheap forward sweep per band stores
 // (S, window) once per LDS-staged segment, one per segment stores them every kChunk
 // rows in LDS, and each chunk is then replayed forward into registers and
-// walked backwards.  The windowed sum of b*overflow lives in a ring of W+1
-// rows in global memory that is touched only while some overflow term of the
-// wave is above `tail_threshold` (long near-exact matches).
+// walked backwards.  The windowed sum of b*overflow takes its leaving terms from a
+// ring in global memory that is touched only while some overflow term of the wave is
+// above `tail_threshold` (long near-exact matches).
 //
 // Each chunk leaves its route weights d*p and gate adjoints h in LDS as
 // [row][lane] tiles (with zero margins), from which the three contractions
@@ -1377,6 +1388,7 @@ void vjp_gradients_kernel(VjpParams P) {
   // dQ and dK are linear in the route adjoints, so the constant factor of every adjoint
   // (adjoint_gain) is applied here, once per flushed element, instead of once per pair
   const float symbol_scale = -0.5f * P.mismatch_scale / static_cast<float>(D) * adjoint_gain;
+  constexpr int kUnreadRows = PIECES ? 1 : 0;  // behind the ring's last row
   float* ring = P.block_scratch +
       (static_cast<int64_t>(blockIdx.x) * NW + wave) * P.block_scratch_floats;
   // without chunk records: (S, window) before every chunk of the current segment, then
@@ -1384,8 +1396,9 @@ void vjp_gradients_kernel(VjpParams P) {
   // (three-term form) what the float32 ring terms do not hold of (b + rest) * overflow, as
   // bfloat16: the second float of the windowed sum
   [[maybe_unused]] uint16_t* ring_low =
-      reinterpret_cast<uint16_t*>(ring + static_cast<int64_t>(P.ring_rows) * kWave);
-  float* ck_evidence = ring + static_cast<int64_t>(P.ring_rows) * (kWave + kWave / 2);  // [SEG_CHUNKS][64]
+      reinterpret_cast<uint16_t*>(ring + static_cast<int64_t>(P.ring_rows + kUnreadRows) * kWave);
+  float* ck_evidence =
+      ring + static_cast<int64_t>(P.ring_rows + kUnreadRows) * (kWave + kWave / 2);  // [SEG_CHUNKS][64]
   int* ck_window = reinterpret_cast<int*>(ck_evidence + SEG_CHUNKS * kWave);
   // without records, two levels of (S, window) checkpoints: before every group of
   // `segment_group` segments of the band (one forward sweep over the band), and before every
@@ -2112,11 +2125,22 @@ void vjp_gradients_kernel(VjpParams P) {
             }
             const bool any_term = __ballot(term != 0.0f) != 0ull;
             if (any_term) {
-              if (ring_live == 0) ring_fresh = P.ring_rows;
-              ring_live = P.ring_rows;
+              const int window_rows = PIECES ? W + 1 : P.ring_rows;
+              if (ring_live == 0) ring_fresh = window_rows;
+              ring_live = window_rows;
             }
             if (ring_live > 0) {
-              const int slot = i % P.ring_rows;
+              // slots of this row and of row i + W + 1, which leaves the window: the same one in a
+              // ring of W + 1 rows, which whole bands have.  In a shorter one the row behind the
+              // last takes the terms of rows that the walk does not leave again (a branch around
+              // the store cost a fifth of the pass where every window is full of matches).
+              int own_slot = i % P.ring_rows;
+              int slot = own_slot;
+              if constexpr (PIECES) {
+                slot += P.ring_skip;
+                if (slot >= P.ring_rows) slot -= P.ring_rows;
+                if (i - W - 1 < row_begin) own_slot = P.ring_rows;
+              }
               float leaving = 0.0f;
               [[maybe_unused]] float leaving_low = 0.0f;
               if (ring_fresh > 0) {
@@ -2127,13 +2151,13 @@ void vjp_gradients_kernel(VjpParams P) {
                   leaving_low = __uint_as_float(uint32_t(ring_low[slot * kWave + lane]) << 16);
                 }
               }
-              ring[slot * kWave + lane] = term;
+              ring[own_slot * kWave + lane] = term;
               if constexpr (TERMS == 2) {
                 ring_sum += term - leaving;
               } else {
                 // the low part enters the sum as it is stored, so that it leaves as it entered
                 const uint32_t low_bits = __float_as_uint(term_low) & 0xffff0000u;
-                ring_low[slot * kWave + lane] = static_cast<uint16_t>(low_bits >> 16);
+                ring_low[own_slot * kWave + lane] = static_cast<uint16_t>(low_bits >> 16);
                 const float added = __fadd_rn(ring_sum, term);
                 const float added_rest = __fsub_rn(term, __fsub_rn(added, ring_sum));
                 const float left = __fsub_rn(added, leaving);

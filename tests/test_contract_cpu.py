@@ -289,6 +289,28 @@ def test_backward_workspace_sizes_at_training_shapes():
         cabi.set_record_budget(None)
 
 
+@pytest.mark.parametrize("B,T,N,S,H,W,most_mib", [
+    # one head or two, windows from an eighth of the sequence to all of it: twice what whole bands
+    # took with a ring of W + 1 rows each (7, 101, 50, 26 and 223 MiB)
+    (1, 2048, 0, 0, 1, 256, 16), (1, 4096, 0, 0, 1, 4096, 202), (1, 2048, 0, 0, 2, 2048, 101),
+    (1, 2048, 0, 0, 2, 1024, 53), (1, 4096, 0, 0, 8, 1024, 470),
+    # packed: as many rings as waves, since the lengths that decide how many pieces there are are
+    # on the device, but rings of the longest piece these may ask for (160 and 64 rows)
+    (0, 0, 4096, 2, 2, 1024, 2048 * 176 * 384 / 2 ** 20 + 24),
+    (0, 0, 2048, 2, 2, 256, 2048 * 80 * 384 / 2 ** 20 + 12),
+])
+def test_the_scratch_of_pieces_is_that_of_the_rows_they_walk(B, T, N, S, H, W, most_mib):
+    """The gradient kernel's ring holds the overflow terms that leave the window again while a wave
+    walks: pieces need little more than their own rows, windows near the sequence next to none.
+    A ring of W + 1 rows for every piece took 106 to 1 638 MiB at these shapes."""
+
+    problem = cabi.RosaProblem(dtype=0, B=B, T=T, N=N or B * T, S=S, H=H, D=8, Hv=H, Dv=8, W=W)
+    if S:
+        problem.cu_seqlens = 1  # any non-null address: the size query never dereferences it
+    size = cabi.load().rosa_hip_vjp_workspace_bytes(ctypes.byref(problem), 7, 1.0, 0)
+    assert size <= most_mib * 2 ** 20
+
+
 def test_gradient_launch_plan_follows_the_shape():
     """Host arithmetic of the gradient kernel's launch form (no device call): blocks of two
     waves where the tiles are wide and bands outnumber the resident waves, the row queue

@@ -664,6 +664,40 @@ def test_bands_cut_into_pieces_match_oracle(cabi, c_oracle, records, B, T, H, D,
         assert_gradients_close(got, unsplit.cpu(), name + " against whole bands", slack)
 
 
+@pytest.mark.parametrize("records", [True, False], ids=["records", "no_records"])
+@pytest.mark.parametrize("T,W,piece_rows,two_waves,pattern,ms", [
+    (300, 148, -1, False, "all_match", 3.0), (300, 149, -1, False, "all_match", 3.0),
+    (300, 150, -1, True, "all_match", 3.0), (300, 200, -1, True, "periodic", 3.0),
+    (300, 297, -1, False, "all_match", 3.0), (300, 298, -1, False, "periodic", 3.0),
+    (300, 299, -1, True, "all_match", 3.0),
+    (420, 33, 64, False, "all_match", 3.0), (420, 79, 64, False, "all_match", 3.0),
+    (420, 80, 64, False, "periodic", 3.0), (420, 81, 64, False, "all_match", 3.0),
+    (420, 300, 96, False, "all_match", 3.0), (420, 50, 64, False, "random", 0.05),
+])
+def test_overflow_terms_leave_rings_shorter_than_the_window(cabi, c_oracle, records, T, W, piece_rows,
+                                                            two_waves, pattern, ms):
+    """Windows around half the sequence, around the sequence and around a piece and its halo: where
+    the ring of overflow terms stops being W + 1 rows.  Every window is full of matches, so that
+    every row's term enters the sum and leaves it again."""
+
+    query, key, value, grad_output = make_case(1, T, 2, 6, 1, 8, torch.float32, seed=T + W,
+                                               pattern=pattern)
+    cabi.set_gradient_piece_rows(piece_rows)
+    cabi.set_gradient_block_waves(2 if two_waves else None)
+    cabi.set_record_budget(None if records else 0)
+    try:
+        *_, grads = run_device(cabi, query, key, value, grad_output, W, ms=ms)
+    finally:
+        cabi.set_gradient_piece_rows(None)
+        cabi.set_gradient_block_waves(None)
+        cabi.set_record_budget(None)
+    want = c_oracle.surrogate_vjp(query, key, value, grad_output, max_suffix_length=W,
+                                  mismatch_scale=ms)
+    slack = max(1.0, 2.4142 * ((1.0 + min(W, T)) ** 0.5 - 1.0) / 40.0)
+    for name, got, expected in zip(("grad_query", "grad_key", "grad_value"), grads, want):
+        assert_gradients_close(got, expected, name, slack)
+
+
 def query_gradient_of_any_range(query, key, value, grad_output, W, ms):
     """dQ of one sequence and head in float64, every adjoint's share of a row as a sum of positive
     products (the streamed oracle takes the tail of a score by subtraction, which loses shares
