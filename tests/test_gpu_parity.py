@@ -291,6 +291,29 @@ def test_packed_layout_matches_oracle(cabi, c_oracle, block_waves, lengths, H, D
             assert torch.count_nonzero(grads[0][start]) == 0
 
 
+@pytest.mark.parametrize("count", [1, 2, 63, 64, 65, 255, 256, 257, 700])
+def test_packed_tables_of_many_sequences_match_oracle(cabi, c_oracle, count):
+    """The tables of a packed batch come from one block of 256 threads, four waves with a scan
+    each: a sequence per thread, edges of waves, several sequences per thread; empty ones, ones of
+    a token, one that is cut into pieces, at every place."""
+
+    rng = np.random.default_rng(count)
+    lengths = rng.integers(0, 9, count)
+    lengths[rng.integers(0, count, 3)] = (70, 131, 1)
+    lengths[-1] = max(lengths[-1], 2)
+    offsets = [0] + [int(x) for x in np.cumsum(lengths)]
+    query, key, value, grad_output = (
+        t[0] for t in make_case(1, offsets[-1], 2, 3, 1, 4, seed=count, pattern="shifted"))
+    out, _, _, _, grads = run_device(cabi, query, key, value, grad_output, 20, p=0.1, seed=5,
+                                     cu_seqlens=offsets)
+    want_out, _ = c_oracle.varlen_hard_forward(query, key, value, offsets, 20)
+    assert torch.equal(out.cpu(), want_out)
+    want = c_oracle.varlen_surrogate_vjp(query, key, value, offsets, grad_output,
+                                         max_suffix_length=20, dropout_p=0.1, seed=5)
+    for name, got, expected in zip(("grad_query", "grad_key", "grad_value"), grads, want):
+        assert_gradients_close(got, expected, name)
+
+
 def test_packed_equals_dense_batch_with_same_seed(cabi):
     # reference tests/test_soft_varlen.py:304-389
     B, T, H, D, Hv, Dv = 3, 70, 2, 4, 1, 5
