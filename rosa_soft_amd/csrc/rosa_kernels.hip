@@ -1353,9 +1353,13 @@ int64_t band_rows_at_most(const Layout& L) {
 }
 
 // Up to this many rows per resident wave the gradient pass runs as its three-term form alone,
-// which serves every input: below it the launch that returns at once would cost more than
-// the third term.
-constexpr int kSingleFormRows = 64;
+// which serves every input: there the second launch, which finds that it does not apply, costs as
+// much as the third term.  Measured at 2 to 200 rows per wave: where some match is long the one
+// form saves 4 us (2 rows 36.6 -> 32.2, 25 rows 50.6 -> 46.6, 100 rows 89.5 -> 85.9, 200 rows
+// 129.3 -> 125.2), where none is it costs 1.5 us at 2 to 25 rows (41.0 -> 42.5, 45.6 -> 47.2), 3 at
+// 50 (54.5 -> 57.9), 4 at 100 (137.4 -> 142.5, 32 values) and 10 at 200 (109.2 -> 118.9).  A packed
+// batch counts as one sequence: nothing larger runs the third term for nothing.
+constexpr int kSingleFormRows = 96;
 
 // How the gradient kernel is launched for a tile shape: waves per block, whether row tiles
 // are queued between the bands of a block, and the LDS of a block.
