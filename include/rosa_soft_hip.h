@@ -87,10 +87,12 @@ void rosa_hip_set_gradient_block_waves(int waves);
 
 /*
  * Rows of a piece of a diagonal band in the backward's gradient kernel: 0 for the library's
- * choice by shape (the default: bands are cut only when there are fewer than two of them per
- * resident wave, into pieces of at least four windows), -1 for never, or a number of rows
- * (rounded up to whole 32-row segments, at least 64).  Pieces of one band are walked by
- * different waves, each starting max_suffix_length - 1 rows below its last row.  No
+ * choice by shape (the default: with fewer than two bands per resident wave, bands longer than
+ * a tenth above a wave's share of all rows are cut into pieces of that many, at least 32), -1
+ * for never, or a number of rows (rounded up to whole 32-row segments, at least 64).  Pieces of
+ * one band are walked by different waves, each starting as many 16-row chunks below its last
+ * row as hold max_suffix_length - 1 rows, or fewer where the match gates of every diagonal
+ * multiply to so little that no float32 carry survives them.  No
  * counterpart in the reference; the knob exists for measurements and so that tests can
  * force cuts on small problems.  Like the other setters it must not race with size queries
  * or launches of other threads.
@@ -123,10 +125,21 @@ int rosa_hip_gradient_block_plan(const rosa_problem* problem, int* waves, int* r
 /*
  * Whether and how the gradient kernel will cut the diagonal bands of `problem` into pieces
  * (no counterpart in the reference; see rosa_hip_set_gradient_piece_rows): `piece_rows` is
- * the length of a piece in rows, 0 for whole bands, `pieces` the work items per band.  Host
- * arithmetic only; returns 0 or a problem-check status.
+ * the length of a piece in rows, 0 for whole bands, `pieces` the work items of the longest
+ * band.  Host arithmetic only; returns 0 or a problem-check status.  Of a packed problem this
+ * is the plan of S equal sequences, by which the form of the kernel is chosen; how long its
+ * pieces are is decided on the device, by the lengths: rosa_hip_packed_piece_plan.
  */
 int rosa_hip_gradient_piece_plan(const rosa_problem* problem, int* piece_rows, int* pieces);
+
+/*
+ * The same for a packed problem whose S + 1 offsets the caller holds in host memory (no
+ * counterpart in the reference): what the device will decide by them.  `piece_rows` is 0 for
+ * whole bands, `items` the work items of all bands of all heads; either may be NULL.  Host
+ * arithmetic only.
+ */
+int rosa_hip_packed_piece_plan(const rosa_problem* problem, const int32_t* host_offsets,
+                               int* piece_rows, int64_t* items);
 
 /*
  * Measurement aid, no counterpart in the reference: the rate at which this GPU performs

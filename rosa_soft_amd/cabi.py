@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "rosa_hip_measure_atomic_rate",
     "rosa_hip_gradient_block_plan",
     "rosa_hip_gradient_piece_plan",
+    "rosa_hip_packed_piece_plan",
     "rosa_hip_hard_forward",
     "rosa_hip_hard_routes",
     "rosa_hip_hard_forward_bits",
@@ -144,6 +145,11 @@ def load() -> ctypes.CDLL:
     library.rosa_hip_gradient_piece_plan.restype = ctypes.c_int
     library.rosa_hip_gradient_piece_plan.argtypes = [
         problem_p, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int),
+    ]
+    library.rosa_hip_packed_piece_plan.restype = ctypes.c_int
+    library.rosa_hip_packed_piece_plan.argtypes = [
+        problem_p, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int),
+        ctypes.POINTER(ctypes.c_int64),
     ]
     library.rosa_hip_measure_atomic_rate.restype = ctypes.c_int
     library.rosa_hip_measure_atomic_rate.argtypes = [
@@ -666,7 +672,8 @@ def set_forward_index(mode: Optional[str]) -> None:
 def gradient_block_plan(query: Tensor, value: Tensor, max_suffix_length: int,
                         cu_seqlens: Optional[Tensor] = None) -> dict:
     """Launch form of the gradient kernel for a problem: waves per block, row queue, LDS bytes,
-    and the rows of a piece of a band (0: whole bands) with the work items per band."""
+    and the rows of a piece of a band (0: whole bands) with the work items of the longest band.
+    The cut of a packed batch depends on its lengths: offsets on the device are read back."""
 
     problem = make_problem(query, value, max_suffix_length, cu_seqlens)
     waves, queue, lds = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_size_t(0)
@@ -677,6 +684,14 @@ def gradient_block_plan(query: Tensor, value: Tensor, max_suffix_length: int,
     status = load().rosa_hip_gradient_piece_plan(
         ctypes.byref(problem), ctypes.byref(piece_rows), ctypes.byref(pieces))
     _check(status, "rosa_hip_gradient_piece_plan")
+    if cu_seqlens is not None:
+        offsets = cu_seqlens.to(device="cpu", dtype=torch.int32).contiguous()
+        status = load().rosa_hip_packed_piece_plan(
+            ctypes.byref(problem), ctypes.cast(offsets.data_ptr(), ctypes.POINTER(ctypes.c_int32)),
+            ctypes.byref(piece_rows), None)
+        _check(status, "rosa_hip_packed_piece_plan")
+        longest = int((offsets[1:] - offsets[:-1]).max())
+        pieces.value = max(1, -(-(longest - 1) // piece_rows.value)) if piece_rows.value else 1
     return dict(waves=waves.value, row_queue=bool(queue.value), lds_bytes=lds.value,
                 piece_rows=piece_rows.value, pieces=pieces.value)
 

@@ -90,6 +90,15 @@ struct PieceLimits {
   int32_t* stats_prefix;
 };
 
+// Rows of a piece of the gradient pass over a packed batch, by its lengths: on the device, where
+// prepare_sequences_kernel decides, and on the host for callers that hold the lengths.
+__host__ __device__ inline int packed_gradient_piece_rows(int forced_rows, int64_t band_rows,
+                                                          int64_t bands, int longest,
+                                                          int64_t waves) {
+  if (forced_rows != 0) return forced_rows > 0 ? forced_rows : 0;
+  return piece_rows_for(band_rows, bands, longest, waves, kPieceRowsMin, kPieceAlign);
+}
+
 // Exclusive prefix sums over the threads of a block, and the totals, of COUNT values at once: a
 // scan per wave and one round through LDS.
 constexpr int kPrepareThreads = 256;
@@ -175,9 +184,8 @@ __global__ __launch_bounds__(kPrepareThreads) void prepare_sequences_kernel(
 
   // index space of the chunk records, and the pieces of the bands
   const int64_t all_rows = totals[1] * H, bands = totals[0] * H;
-  const int forced = pieces.forced_gradient_rows;
-  const int gradient_rows = forced != 0 ? max(forced, 0)
-      : piece_rows_for(all_rows, bands, longest, pieces.gradient_waves, kPieceRowsMin, kPieceAlign);
+  const int gradient_rows = packed_gradient_piece_rows(pieces.forced_gradient_rows, all_rows, bands,
+                                                       longest, pieces.gradient_waves);
   const int stats_rows =
       piece_rows_for(all_rows, bands, longest, pieces.stats_waves, kPieceRowsMin, kChunk);
   int64_t items[2] = {0, 0}, all_items[2];
@@ -2140,6 +2148,12 @@ bool analytic_reference_is_safe(const Layout& L, float scale) {
   return (bound - kNullScore * scale) * kLog2e < 80.0f;
 }
 
+// rows of a piece that the caller has set for packed batches (rosa_hip_set_gradient_piece_rows)
+int forced_packed_piece_rows(const GradientPlan& plan) {
+  const int forced = g_gradient_piece_rows.load(std::memory_order_relaxed);
+  return forced > 0 ? plan.piece_rows : forced;
+}
+
 template <int DTYPE>
 int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, const void* key,
             const void* value, const void* grad_output, const int32_t* packed_query,
@@ -2153,9 +2167,8 @@ int run_vjp(const rosa_problem* p, const ProblemView& view, const void* query, c
     const int dvp = padded_value_width(width);
     const GradientPlan plan = plan_gradients(L, dvp, value_words(width),
                                              grad_term_pitch(view.grad_terms, dvp));
-    const int forced = g_gradient_piece_rows.load(std::memory_order_relaxed);
     const PieceLimits limits{std::min<int64_t>(plan.waves, w.resident_blocks), w.stats_waves,
-                             forced > 0 ? plan.piece_rows : forced,
+                             forced_packed_piece_rows(plan),
                              w.stats_items_most, at<int32_t>(workspace, w.gradient_prefix),
                              at<int32_t>(workspace, w.stats_prefix)};
     launch_prepare_sequences(p, L, workspace, w.seq_start, w.seq_len, w.block_prefix, w.header,
@@ -3795,6 +3808,43 @@ int rosa_hip_gradient_piece_plan(const rosa_problem* problem, int* piece_rows, i
                                            grad_term_pitch(view.grad_terms, dvp));
   if (piece_rows != nullptr) *piece_rows = plan.piece_rows;
   if (pieces != nullptr) *pieces = plan.max_pieces;
+  return 0;
+}
+
+int rosa_hip_packed_piece_plan(const rosa_problem* problem, const int32_t* host_offsets,
+                               int* piece_rows, int64_t* items) {
+  ProblemView view;
+  const int status = check_problem(problem, &view);
+  if (status != 0) return status;
+  const Layout& L = view.L;
+  if (!L.varlen || host_offsets == nullptr) return fail(1, "a packed problem and its offsets in host memory");
+  bool valid = host_offsets[0] == 0 && host_offsets[L.S] == L.N;
+  for (int s = 0; s < L.S; ++s) valid = valid && host_offsets[s] <= host_offsets[s + 1];
+  if (!valid) return fail(1, "cu_seqlens must start at 0, end at N and never decrease");
+  const int width = std::min(L.Dv, kValueSlice);
+  const int dvp = padded_value_width(width);
+  const GradientPlan plan =
+      plan_gradients(L, dvp, value_words(width), grad_term_pitch(view.grad_terms, dvp));
+  int64_t rows = 0, blocks = 0;
+  int longest = 0;
+  for (int s = 0; s < L.S; ++s) {
+    const int length = host_offsets[s + 1] - host_offsets[s];
+    rows += band_steps_total(length);
+    blocks += (length + 63) / 64;
+    longest = std::max(longest, length);
+  }
+  int cut = 0;
+  if (plan.piece_rows > 0) {  // (else the form that walks whole bands is launched)
+    const VjpWorkspace w = carve_vjp(view, false);
+    cut = packed_gradient_piece_rows(forced_packed_piece_rows(plan), rows * L.H, blocks * L.H, longest,
+                                     std::min<int64_t>(plan.waves, w.resident_blocks));
+  }
+  int64_t pieces = 0;
+  for (int s = 0; s < L.S; ++s) {
+    pieces += pieces_of_sequence(host_offsets[s + 1] - host_offsets[s], cut) * L.H;
+  }
+  if (piece_rows != nullptr) *piece_rows = cut;
+  if (items != nullptr) *items = pieces;
   return 0;
 }
 

@@ -404,6 +404,46 @@ def test_pieces_of_bands_are_planned_for_the_waves_of_the_form_that_walks_them(d
         assert len(found) == 1 and 1024 * found[0]["waves_per_simd"] == waves
 
 
+@pytest.mark.parametrize("lengths,H,forced", [
+    ([1, 37, 129, 513, 1000, 2047, 3001], 12, None), ([3000, 1, 1, 1, 1, 1, 1], 2, None),
+    ([33, 0, 98, 2, 161, 64, 65, 66], 2, None), ([64, 65], 1, 64), ([700, 300, 257], 4, 96),
+    ([8192] * 4, 64, None), ([700, 300], 4, -1),
+])
+def test_the_piece_plan_of_a_packed_batch_is_that_of_its_lengths(lengths, H, forced):
+    """Not that of equal sequences: the work items are the pieces that every band of every
+    sequence really has, and the reported cut is the one that fits them."""
+
+    offsets = torch.zeros(len(lengths) + 1, dtype=torch.int32)
+    offsets[1:] = torch.tensor(lengths).cumsum(0)
+    query = torch.empty(sum(lengths), H, 8)
+    value = torch.empty(sum(lengths), H, 8)
+    problem = cabi.make_problem(query, value, 32, offsets)
+    rows, items = ctypes.c_int(-7), ctypes.c_int64(-7)
+    packed_plan = lambda host: cabi.load().rosa_hip_packed_piece_plan(
+        ctypes.byref(problem), ctypes.cast(host.data_ptr(), ctypes.POINTER(ctypes.c_int32)),
+        ctypes.byref(rows), ctypes.byref(items))
+    cabi.set_gradient_piece_rows(forced)
+    try:
+        assert packed_plan(offsets) == 0
+        plan = cabi.gradient_block_plan(query, value, 32, offsets)
+        broken = offsets.clone()
+        broken[1] = -1
+        assert packed_plan(broken) != 0 and packed_plan(offsets) == 0
+    finally:
+        cabi.set_gradient_piece_rows(None)
+    bands = [n - 1 - 64 * j for n in lengths for j in range((n - 2) // 64 + 1 if n > 1 else 0)]
+    assert plan["piece_rows"] == rows.value
+    if rows.value == 0:
+        assert items.value == H * len(bands) and plan["pieces"] == 1
+        assert forced == -1 or len(bands) * H >= 4096
+    else:
+        assert items.value == H * sum(-(-n // rows.value) for n in bands)
+        assert plan["pieces"] == -(-(max(lengths) - 1) // rows.value)
+        share = 1.1 * H * sum(bands) / 2048
+        assert rows.value == forced or rows.value <= max(32, share + 32)
+        assert rows.value == forced or rows.value >= min(share, max(lengths) // 2)
+
+
 def test_no_kernel_of_the_last_build_spills_or_uses_scratch():
     """The build records what the compiler reported per kernel.  Spilled vector registers and
     scratch memory are performance faults of the backward kernels (a reload waits behind

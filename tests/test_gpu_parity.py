@@ -314,6 +314,28 @@ def test_packed_tables_of_many_sequences_match_oracle(cabi, c_oracle, count):
         assert_gradients_close(got, expected, name)
 
 
+@pytest.mark.parametrize("lengths", [
+    [1, 37, 129, 513, 1000, 2047, 3001], [900], [5] * 300 + [2000], [64, 65, 66, 0, 128, 129, 130],
+])
+def test_the_device_cuts_a_packed_batch_as_the_host_plan_says(cabi, lengths):
+    """Rows of a piece and work items, header words 5 and 6 of the workspace, against
+    rosa_hip_packed_piece_plan and a count of the pieces of every band."""
+
+    offsets = [0] + [int(x) for x in np.cumsum(lengths)]
+    query, key, value, grad_output = (
+        t[0].to(DEVICE) for t in make_case(1, offsets[-1], 3, 4, 1, 4, seed=3))
+    cu_seqlens = torch.tensor(offsets, dtype=torch.int32, device=DEVICE)
+    _, packed_query, packed_key, _ = cabi.hard_forward(query, key, value, 16, cu_seqlens)
+    workspace = torch.empty(cabi.vjp_workspace_bytes(query, value, 16, cu_seqlens),
+                            dtype=torch.uint8, device=DEVICE)
+    cabi.surrogate_vjp(query, key, value, grad_output, packed_query, packed_key, None, 16, 1.0, 0.0,
+                       3.0, 7, cu_seqlens, workspace)
+    rows, items = workspace[20:28].view(torch.int32).tolist()
+    assert rows == cabi.gradient_block_plan(query, value, 16, cu_seqlens)["piece_rows"] > 0
+    bands = [n - 1 - 64 * j for n in lengths for j in range((n - 2) // 64 + 1 if n > 1 else 0)]
+    assert items == 3 * sum(-(-n // rows) for n in bands)
+
+
 def test_packed_equals_dense_batch_with_same_seed(cabi):
     # reference tests/test_soft_varlen.py:304-389
     B, T, H, D, Hv, Dv = 3, 70, 2, 4, 1, 5
