@@ -250,9 +250,9 @@ class RosaRuntime:
         self._query_history: Optional[Tensor] = None    # [S, H, capacity] uint8
         self._key_history: Optional[Tensor] = None      # [S, H, capacity] uint8
         self._payload_history: Optional[Tensor] = None  # [S, Hp, capacity] uint8
-        # the library's description of an update, as far as updates share it; made anew when
-        # the histories it points to are
-        self._update: Optional[cabi.RosaRouterUpdate] = None
+        # the bytes of the library's description of an update, as far as updates share it; made
+        # anew when the histories it points to are
+        self._update: Optional[bytes] = None
         self._last_update = None            # event recorded after the latest update's launches
         self._last_stream = None            # ... and the stream they went to
 
@@ -516,9 +516,8 @@ class RosaRuntime:
             self._device_lengths_next = torch.empty_like(self._device_lengths)
         uniform = offsets is None or min(chunks) == longest_chunk
         tables = None if uniform else torch.tensor(offsets, dtype=torch.int32).to(self._device)
-        update = self._update
-        if update is None:  # what every update has in common until the histories grow
-            update = self._update = cabi.RosaRouterUpdate()
+        if self._update is None:  # what every update has in common until the histories grow
+            update = cabi.RosaRouterUpdate()
             update.S, update.H, update.Hp = self._slot_count, self._num_heads, self._num_payload_heads
             update.W = min(self._max_suffix_length, 2**31 - 1)
             update.qk_bits, update.payload_bits = self._qk_bits, self._payload_bits
@@ -526,6 +525,10 @@ class RosaRuntime:
             update.query_history = self._query_history.data_ptr()
             update.key_history = self._key_history.data_ptr()
             update.payload_history = self._payload_history.data_ptr()
+            self._update = bytes(update)
+        # (a description of its own for every update: the library reads it with the interpreter's
+        # lock released)
+        update = cabi.RosaRouterUpdate.from_buffer_copy(self._update)
         update.tokens = tokens
         update.longest_chunk = longest_chunk
         update.uniform_chunk = longest_chunk if uniform else 0

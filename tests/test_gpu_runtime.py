@@ -344,6 +344,29 @@ def test_updates_on_different_streams_are_serialised(rosa):
     assert torch.equal(torch.cat([r[1] for r in results], dim=1).cpu(), want[1])
 
 
+def test_every_update_owns_the_description_the_library_reads(rosa, monkeypatch):
+    """The library reads it with the interpreter's lock released: an update that another thread
+    starts meanwhile must not change it, whether the histories grow in between or not."""
+
+    from rosa_soft_amd import cabi
+
+    seen, launch = [], cabi.router_update
+
+    def watched(update, *arguments):
+        result = launch(update, *arguments)
+        seen.append((update, bytes(update)))
+        return result
+
+    monkeypatch.setattr(cabi, "router_update", watched)
+    with rosa.RosaRuntime(2, 1, 4, 4, 8) as runtime:
+        for step, tokens in enumerate((3, 1, 1, 400, 1)):
+            symbols = random_packed((2, tokens, 2), 4, step).to(DEVICE)
+            runtime.update_packed(symbols, symbols, symbols[:, :, :1])
+    assert len(seen) == 5
+    for update, as_launched in seen:
+        assert bytes(update) == as_launched
+
+
 @pytest.mark.parametrize("pattern", ["random", "period7", "constant"])
 def test_long_chunks_route_through_the_index_of_the_keys(rosa, pattern):
     # chunks beyond 8 rows on histories of 512 tokens or more take the index of the keys
