@@ -246,6 +246,7 @@ class RosaRuntime:
         self._slots_initialized = False
         self._lengths: list = []            # host mirror of the per-slot history lengths
         self._device_lengths: Optional[Tensor] = None   # [S] int32, advanced by the library
+        self._device_lengths_next: Optional[Tensor] = None
         self._capacity = 0
         self._query_history: Optional[Tensor] = None    # [S, H, capacity] uint8
         self._key_history: Optional[Tensor] = None      # [S, H, capacity] uint8
@@ -413,7 +414,8 @@ class RosaRuntime:
         run_stream = stream if (stream is not None and caller_device == self._device) else None
         done = None
         if run_stream is not None:
-            run_stream.wait_stream(torch.cuda.current_stream(self._device))
+            caller_stream = torch.cuda.current_stream(self._device)
+            run_stream.wait_stream(caller_stream)
         with torch.cuda.stream(run_stream) if run_stream is not None else _NullContext():
             # Updates are serialised whatever streams they are given (the reference's
             # runtime does the same): this one starts after the previous one has finished
@@ -423,6 +425,9 @@ class RosaRuntime:
                 working_stream.wait_event(self._last_update)
             if caller_device != self._device or query.device != self._device:
                 query, key, payload = (tensor.to(self._device) for tensor in (query, key, payload))
+            if run_stream is not None:  # symbols of the caller's stream, which may free them
+                for tensor in (query, key, payload):
+                    tensor.record_stream(run_stream)
             output, ends = self._route(query, key, payload, tokens, chunks, offsets, lead,
                                        working_stream)
             if not return_packed:
@@ -439,6 +444,11 @@ class RosaRuntime:
             if self._last_update is None:
                 self._last_update = torch.cuda.Event()
             self._last_update.record(working_stream)
+            if working_stream != self._last_stream:  # may be freed while this stream reads them
+                for held in (self._query_history, self._key_history, self._payload_history,
+                             self._device_lengths, self._device_lengths_next):
+                    if held is not None:
+                        held.record_stream(working_stream)
             self._last_stream = working_stream
             if caller_device != self._device:
                 output, ends = output.to(caller_device), ends.to(caller_device)
@@ -446,7 +456,7 @@ class RosaRuntime:
                 done = torch.cuda.Event()
                 done.record(run_stream)
                 for tensor in (output, ends):
-                    tensor.record_stream(torch.cuda.current_stream(self._device))
+                    tensor.record_stream(caller_stream)
         work = _RuntimeWork((output, ends), done, run_stream)
         return work if async_op else work.wait()
 

@@ -367,6 +367,35 @@ def test_every_update_owns_the_description_the_library_reads(rosa, monkeypatch):
         assert bytes(update) == as_launched
 
 
+@pytest.mark.parametrize("logits", [True, False])
+def test_tensors_of_an_update_on_a_side_stream_outlive_it(rosa, logits):
+    """The side stream is still busy when the caller drops its inputs, and the runtime its
+    histories: what the caller's stream then allocates and fills must not be their memory."""
+
+    bits, shape = 4, (2, 300, 3)
+    symbols = [random_packed(shape, bits, seed) for seed in (1, 2, 3)]
+    want = expect_dense(*symbols, bits, bits, 16)
+    inputs = [part.to(DEVICE) for part in symbols]
+    if logits:
+        inputs = [((part.unsqueeze(-1) >> torch.arange(bits, device=DEVICE)) & 1).float() - 0.5
+                  for part in inputs]
+    side = torch.cuda.Stream()
+    with rosa.RosaRuntime(3, 3, bits, bits, 16) as runtime:
+        update = runtime.update if logits else runtime.update_packed
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(100_000_000)
+        work = update(*inputs, stream=side, async_op=True, return_packed=True)
+        del inputs
+        runtime.reset()
+        # everything the allocator would hand out again, overwritten while the side stream waits
+        junk = [torch.full((size,), 255, dtype=torch.uint8, device=DEVICE)
+                for size in (2 * 300 * 3, 2 * 300 * 3 * bits * 4, 2 * 3 * 512, 8, 64) for _ in range(12)]
+        output, ends = work.wait()
+        assert torch.equal(output.cpu(), want[0]) and torch.equal(ends.cpu(), want[1])
+        del junk
+
+
 @pytest.mark.parametrize("pattern", ["random", "period7", "constant"])
 def test_long_chunks_route_through_the_index_of_the_keys(rosa, pattern):
     # chunks beyond 8 rows on histories of 512 tokens or more take the index of the keys
