@@ -421,7 +421,8 @@ class RosaRuntime:
             # runtime does the same): this one starts after the previous one has finished
             # with the histories, including a growth copy.
             working_stream = torch.cuda.current_stream(self._device)
-            if self._last_update is not None and working_stream != self._last_stream:
+            other_stream = working_stream != self._last_stream
+            if other_stream and self._last_update is not None:
                 working_stream.wait_event(self._last_update)
             if caller_device != self._device or query.device != self._device:
                 query, key, payload = (tensor.to(self._device) for tensor in (query, key, payload))
@@ -444,7 +445,7 @@ class RosaRuntime:
             if self._last_update is None:
                 self._last_update = torch.cuda.Event()
             self._last_update.record(working_stream)
-            if working_stream != self._last_stream:  # may be freed while this stream reads them
+            if other_stream:  # they may be freed while this stream reads them
                 for held in (self._query_history, self._key_history, self._payload_history,
                              self._device_lengths, self._device_lengths_next):
                     if held is not None:
@@ -542,14 +543,14 @@ class RosaRuntime:
         update.tokens = tokens
         update.longest_chunk = longest_chunk
         update.uniform_chunk = longest_chunk if uniform else 0
-        update.chunk_offsets = None if uniform else tables.data_ptr()
+        if not uniform:
+            update.chunk_offsets = tables.data_ptr()
         update.history_lengths = self._device_lengths.data_ptr()
         update.history_lengths_out = self._device_lengths_next.data_ptr()
         update.query, update.key, update.payload = \
             query.data_ptr(), key.data_ptr(), payload.data_ptr()
         update.output, update.matched_key_end = output.data_ptr(), ends.data_ptr()
         update.longest_total = longest_total
-        update.workspace, update.workspace_bytes = None, 0
         workspace = cabi.router_update(update, self._device, stream)
         # stream-ordered launches: keep what they read alive until they have run
         for held in (tables, workspace):
