@@ -286,7 +286,7 @@ __host__ __device__ inline int64_t checkpoint_slots(int64_t steps, int64_t bands
 // of full ones (gradient pass of 4096 tokens x 8 heads, W 64: 512 rows 241 us, 576 rows 197; of
 // 1500 x 16, 64 values: 256 rows 251 us, 320 rows 189).  Where every band has a wave of its own
 // halves are short enough: the waves that end first are those of the shortest bands, and take the
-// longest second halves (2 x 1024 tokens x 64 heads: 512 rows 210 us, 608 rows 231).
+// longest second halves (2 x 1024 tokens x 64 heads: 512 rows 210 us, 640 rows 237).
 // What a piece walks beyond its own rows (a halo below it or a sweep in front of it, W rows at
 // most) is left out: waves in parallel repeat it, and even where the window is the sequence and
 // every symbol matches, the smallest pieces are the fastest (2048 tokens x 2 heads, W 2048:

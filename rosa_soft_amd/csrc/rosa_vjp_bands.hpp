@@ -84,7 +84,9 @@ constexpr int gradient_ring_rows(int window, int64_t walked) {
 // header words that hold the piece plan of a packed batch
 constexpr int kHeaderGradientPieces = 5;  // rows, then work items in all
 constexpr int kHeaderStatsPieces = 7;
-constexpr int kPieceRowsMin = 32;   // rows of a piece at least
+// rows of a piece at least (with waves to spare, gradient pass of 256 tokens x 4 heads: 32 rows
+// 31 us, 64 rows 47; 2 x 700 tokens x 4 heads: 36 and 42; fewer are less than a staged segment)
+constexpr int kPieceRowsMin = 32;
 constexpr int kPieceAlign = 32;     // pieces of the gradient pass are whole staged segments
 
 // Terms of the bfloat16 expansion of a float: x = t0 + t1 + t2 exactly (each term is the

@@ -323,10 +323,10 @@ def test_gradient_launch_plan_follows_the_shape():
 
     metric = plan(torch.float32, (2, 4096, 64), 8, 16, 8, 128)
     assert metric["waves"] == 1 and not metric["row_queue"]
-    # 8 192 bands on 3 072 resident waves: whole bands
+    # 8 192 bands, two or more for every wave of the form that walks pieces (2 048): whole bands
     assert metric["piece_rows"] == 0 and metric["pieces"] == 1
-    # configuration 4: 2 048 bands of up to 8 191 rows on 2 048 resident waves are cut into two
-    # pieces of whole 32-row segments, each at least four windows long
+    # configuration 4: 2 048 bands of up to 8 191 rows on 2 048 resident waves are cut into halves,
+    # whole 32-row segments each
     long_bands = plan(torch.float16, (1, 8192, 16), 2, 16, 32, 256)
     assert long_bands["waves"] == 1 and long_bands["pieces"] == 2
     assert long_bands["piece_rows"] == 4096 and long_bands["piece_rows"] >= 4 * 256

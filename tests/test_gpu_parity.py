@@ -667,8 +667,8 @@ PIECE_CASES = [
 def test_bands_cut_into_pieces_match_oracle(cabi, c_oracle, records, B, T, H, D, Hv, Dv, W, p,
                                             dtype, pattern, piece_rows, mask, lengths):
     """The gradient kernel cuts long bands into pieces when a shape has few of them; forced
-    here at test sizes.  A piece restarts the reverse recurrences W - 1 rows below its last
-    row and leaves its first 64 columns' partial sums to the piece above: long matches that
+    here at test sizes.  A piece restarts the reverse recurrences up to W - 1 rows below its last
+    row (all of them where matches are long, as here) and leaves its first 64 columns' partial sums to the piece above: long matches that
     cross every cut are the cases that would show a wrong halo or a lost partial sum."""
 
     seed = 31337 if p > 0 else None
