@@ -287,6 +287,9 @@ __host__ __device__ inline int64_t checkpoint_slots(int64_t steps, int64_t bands
 // 1500 x 16, 64 values: 256 rows 251 us, 320 rows 189).  Where every band has a wave of its own
 // halves are short enough: the waves that end first are those of the shortest bands, and take the
 // longest second halves (2 x 1024 tokens x 64 heads: 512 rows 210 us, 640 rows 237).
+// Bands that would lose less than a sixteenth stay whole, with the registers of the form for whole
+// bands (4096 tokens, W 64: 56 heads cut at 4032 rows 1084 us, whole 1025; 48 heads cut at 3456 rows
+// 995, whole 1006; 26 heads of 64 values cut at 3744 rows 1221, whole 1298).
 // What a piece walks beyond its own rows (a halo below it or a sweep in front of it, W rows at
 // most) is left out: waves in parallel repeat it, and even where the window is the sequence and
 // every symbol matches, the smallest pieces are the fastest (2048 tokens x 2 heads, W 2048:
@@ -297,7 +300,7 @@ __host__ __device__ inline int piece_rows_for(int64_t band_rows, int64_t bands, 
   if (bands <= capacity && ideal > longest / 2) ideal = longest / 2;
   if (ideal < least) ideal = least;
   const int64_t rows = (ideal + align - 1) / align * align;
-  return rows < longest - 1 ? static_cast<int>(rows) : 0;
+  return 16 * rows <= 15 * static_cast<int64_t>(longest - 1) ? static_cast<int>(rows) : 0;
 }
 
 __host__ __device__ inline int pieces_of_band(int piece_rows, int longest) {

@@ -1433,7 +1433,8 @@ int64_t resident_gradient_waves(const GradientBlockPlan& block, int dvp, int sym
 // as its longest one).  A piece is a whole number of staged segments; piece_rows_for says how long.
 // The waves are those of the form that walks pieces: counted as the whole-band form's, three per
 // SIMD instead of two, 2 x 1024 tokens x 64 heads ran in one and a half rounds of 352-row pieces,
-// 270 us, now in one of 512-row pieces, 210.
+// 270 us, now in one of 512-row pieces, 210; and 4096 tokens x 80 heads were cut, 1781 us, where
+// whole bands at three waves take 1261.
 struct GradientPlan {
   GradientBlockPlan block;
   int piece_rows;   // 0: whole bands
@@ -1477,6 +1478,8 @@ GradientPlan plan_gradients(const Layout& L, int dvp, int value_words_per_column
   plan.waves = piece_waves;
   // The work items, and the rows a piece walks: its own and a halo of whole chunks below it.  The
   // lengths of a packed batch may ask for pieces of up to what one sequence of all tokens would.
+  // (A band that stays whole, a sixteenth longer at most, has no halo: its ring needs W + 1 rows,
+  // or where the window is longer than a piece fewer than that halo leaves room for.)
   int longest_piece = rows;
   if (!L.varlen) {
     plan.items = pieces_of_sequence(L.T, rows) * L.B * L.H;
